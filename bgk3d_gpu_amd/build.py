@@ -16,6 +16,8 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -26,7 +28,7 @@ INCLUDE = PKG.parent / "include"
 ARCH = os.environ.get("BGK_OFFLOAD_ARCH", "gfx950")
 
 COMMON = [
-    "-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",
+    "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{INCLUDE}",
@@ -36,7 +38,8 @@ TARGETS = {
     "libbgk3d_gpu_sp.so": (["v1_abi.hip"], []),
     "libbgk3d_gpu_dp.so": (["v1_abi.hip"], ["-DBGK_DOUBLE"]),
 }
-ENGINE_SOURCES = ["engine.hip", "serving.hip"]
+ENGINE_SOURCES = ["engine.hip", "serving.hip", "launch_f32.hip", "launch_f64.hip", "launch_f16.hip", "launch_bf16.hip",
+                  "launch_mixed1.hip", "launch_mixed2.hip"]
 if (CSRC / "engine.hip").exists():
     TARGETS["libbgk3d_engine.so"] = (ENGINE_SOURCES, [])
 
@@ -48,11 +51,7 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found: the HIP libraries cannot be built")
 
 
-def build_one(name: str, sources, extra, verbose=False) -> Path:
-    LIBDIR.mkdir(parents=True, exist_ok=True)
-    out = LIBDIR / name
-    tmp = out.with_suffix(".so.tmp")
-    cmd = [hipcc(), *COMMON, *extra, *[str(CSRC / s) for s in sources], "-o", str(tmp)]
+def _hipcc(cmd, name, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -61,7 +60,21 @@ def build_one(name: str, sources, extra, verbose=False) -> Path:
         raise RuntimeError(f"hipcc failed for {name}:\n{errs}")
     if errs.strip() and verbose:
         print(errs, file=sys.stderr)
-    os.replace(tmp, out)
+
+
+def build_one(name: str, sources, extra, verbose=False) -> Path:
+    """Compile the sources side by side and link them."""
+    LIBDIR.mkdir(parents=True, exist_ok=True)
+    out = LIBDIR / name
+    with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor(max_workers=8) as ex:
+        objs = [f"{tmp}/{Path(s).stem}.o" for s in sources]
+        jobs = [ex.submit(_hipcc, [hipcc(), *COMMON, *extra, "-c", str(CSRC / s), "-o", o], f"{name}: {s}", verbose)
+                for s, o in zip(sources, objs)]
+        for j in jobs:
+            j.result()
+        lib = out.with_suffix(".so.tmp")
+        _hipcc([hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", str(lib)], name, verbose)
+        os.replace(lib, out)
     return out
 
 
@@ -75,7 +88,6 @@ def build_fortran(verbose=False):
     out = src / "bin"
     out.mkdir(exist_ok=True)
     built = []
-    import tempfile
     for prec, define in (("sp", []), ("dp", ["-DDOUBLE_P"])):
         with tempfile.TemporaryDirectory() as tmp:
             steps = [
@@ -97,8 +109,6 @@ def build_fortran(verbose=False):
 
 
 def build_all(verbose=False):
-    from concurrent.futures import ThreadPoolExecutor
-
     with ThreadPoolExecutor(max_workers=len(TARGETS)) as ex:
         futs = [ex.submit(build_one, n, s, e, verbose) for n, (s, e) in TARGETS.items()]
         libs = [f.result() for f in futs]

@@ -191,80 +191,13 @@ int upload_state(bgk_handle& h)
     if (c.boundary == BGK_BC_INFLOW) {
         for (int buf = 0; buf < 2; ++buf) {
             Lattice19<S> L;
-            for (int d = 0; d < 19; ++d) L.p[d] = d == 18 ? h.arr<S>(0, 18) : h.arr<S>(buf, d);
+            for (int d = 0; d < 19; ++d) L.p[d] = h.arr<S>(d == 18 ? 0 : buf, d);
             hipLaunchKernelGGL(inflow_halo<S>, dim3(ceil_div((long)(c.m + 2) * (c.n + 2), 256)), dim3(256), 0,
                                h.stream, L, h.geom(), (C)h.u_inflow);
         }
         ENG_HIP(hipStreamSynchronize(h.stream));
     }
     return 0;
-}
-
-template <typename S, int BX, int BY, int BZ, bool OB, int FM, int SR>
-void launch_fused(bgk_handle& h)
-{
-    const FusedArgs<S> p = fused_args<S>(h, h.cur);
-    if (h.compact) {
-        hipLaunchKernelGGL((collide_compact<S, BX, BY, BZ, OB, FM, SR>),
-                           dim3((unsigned)ceil_div(p.lend, 256), (unsigned)p.n), dim3(256), compact_lds_cap<S>(),
-                           h.stream, p);
-        return;
-    }
-    const RowMap rm = row_map(p.l);
-    if constexpr (sizeof(S) == 2) {
-        if (p.lend <= p.l) {
-            hipLaunchKernelGGL((collide_fused<S, BX, BY, BZ, OB, FM, SR, false>), fused_grid(rm, p.m, p.n),
-                               fused_block(rm), 0, h.stream, p, rm);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((collide_fused<S, BX, BY, BZ, OB, FM, SR>), fused_grid(rm, p.m, p.n), fused_block(rm), 0,
-                       h.stream, p, rm);
-}
-
-// L = 4 selects the Smagorinsky LES relaxation (FMODE bit 2)
-template <typename S, int SR, int L>
-void dispatch_fused_les(bgk_handle& h)
-{
-    const bgk_config& c = h.cfg;
-    switch (c.boundary) {
-        case BGK_BC_DRIVEN: launch_fused<S, AX_WALL, AX_WALL, AX_LID, false, L, SR>(h); break;
-        case BGK_BC_PERIODIC:
-            if (h.has_obs)
-                launch_fused<S, AX_PERIODIC, AX_PERIODIC, AX_PERIODIC, true, L, SR>(h);
-            else
-                launch_fused<S, AX_PERIODIC, AX_PERIODIC, AX_PERIODIC, false, L, SR>(h);
-            break;
-        case BGK_BC_CHANNEL:
-            if (c.wall_axis == 2) {  // walls at y = 1, m; x and z periodic
-                if (c.force_axis == 3)
-                    launch_fused<S, AX_PERIODIC, AX_WALL, AX_PERIODIC, false, 3 | L, SR>(h);
-                else
-                    launch_fused<S, AX_PERIODIC, AX_WALL, AX_PERIODIC, false, 1 | L, SR>(h);
-            } else if (c.force_axis == 2) {
-                launch_fused<S, AX_PERIODIC, AX_PERIODIC, AX_WALL, false, 2 | L, SR>(h);
-            } else if (c.force_axis == 3) {
-                launch_fused<S, AX_PERIODIC, AX_PERIODIC, AX_WALL, false, 3 | L, SR>(h);
-            } else {
-                launch_fused<S, AX_PERIODIC, AX_PERIODIC, AX_WALL, false, 1 | L, SR>(h);
-            }
-            break;
-        default:
-            if (h.has_obs)
-                launch_fused<S, AX_HALO, AX_PERIODIC, AX_PERIODIC, true, L, SR>(h);
-            else
-                launch_fused<S, AX_HALO, AX_PERIODIC, AX_PERIODIC, false, L, SR>(h);
-            break;
-    }
-}
-
-template <typename S, int SR>
-void dispatch_fused(bgk_handle& h)
-{
-    if (h.cfg.les)
-        dispatch_fused_les<S, SR, 4>(h);
-    else
-        dispatch_fused_les<S, SR, 0>(h);
 }
 
 // Whether this handle's compact collide writes the inflow boundary's x
@@ -276,25 +209,26 @@ bool collide_fills_faces(const bgk_handle& h)
     return h.cfg.les ? kFillsInflowFaces<S, 4> : kFillsInflowFaces<S, 0>;
 }
 
-// queue the boundary work and the fused collide of one step, then swap.
-// `first`: the first step of a stepping call, after which the lattice may
-// have been set or restored -- the outflow kernel then runs whatever the
-// collide writes.
+// queue the boundary work and the fused collide of one step, or of two in
+// one pass where that is faster and two are left, then swap; returns the
+// steps taken.  `first`: the first launch of a stepping call, after which
+// the lattice may have been set or restored -- the outflow kernel then runs
+// whatever the collide writes.
 template <typename S>
-void one_step(bgk_handle& h, hipEvent_t pre, hipEvent_t post, bool first)
+int one_launch(bgk_handle& h, int left, hipEvent_t pre, hipEvent_t post, bool first)
 {
-    if (h.cfg.boundary == BGK_BC_INFLOW && (first || !collide_fills_faces<S>(h))) {
+    const bool pair = h.pair && left >= 2;
+    if (h.cfg.boundary == BGK_BC_INFLOW && (first || pair || !collide_fills_faces<S>(h))) {
         hipLaunchKernelGGL(outflow_halo<S>, dim3(ceil_div((long)h.cfg.m * h.cfg.n, 256)), dim3(256), 0, h.stream,
                            h.current<S>(), h.geom(), h.compact, (typename Storage<S>::compute)h.u_inflow);
     }
     if (pre) (void)hipEventRecord(pre, h.stream);
-    if (h.cfg.rounding && sizeof(S) == 2)
-        dispatch_fused<S, 1>(h);
-    else
-        dispatch_fused<S, 0>(h);
+    launch_step<S>(h, pair);
     if (post) (void)hipEventRecord(post, h.stream);
     h.cur = 1 - h.cur;
-    ++h.steps;
+    if (pair) h.rest = 1 - h.rest;
+    h.steps += pair ? 2 : 1;
+    return pair ? 2 : 1;
 }
 
 // Fortran sequential unformatted records: a 4-byte length, the data, the
@@ -374,9 +308,13 @@ int handle_setup(bgk_handle& h, const bgk_config& c)
     h.nz = c.n + 2;
     // Rows padded to whole lines, or compact rows where those measured
     // faster (prefer_compact: enough of a row's last line unused, or, with
-    // 32/64-bit storage, a lattice of 2^24 cells or more).
+    // 32/64-bit storage, a lattice of 2^24 cells or more).  Lattices that
+    // take two steps per launch keep padded rows: the tiles of collide_pair
+    // start and end on lines (413 against 346 us per FP32 step at 256^3 over
+    // compact rows).
     const double waste = (double)(round_up(c.l, h.A) - c.l) / (double)c.l;
-    h.compact = c.layout == 2 || (c.layout == 0 && prefer_compact(c, waste));
+    h.pair = prefer_pair(c, round_up(c.l + 2, h.A) * h.ny, h.pgrid);
+    h.compact = c.layout == 2 || (c.layout == 0 && !h.pair && prefer_compact(c, waste));
     if (h.compact) {
         // cell (0, 1, k) of every population plane on a line start
         h.nx = c.l + 2;
@@ -559,7 +497,7 @@ int bgk_step(bgk_handle* h, int nsteps)
     if (!h || nsteps < 0) return fail(BGK_EINVAL, "bad arguments");
     ENG_HIP(hipSetDevice(h->cfg.device));
     return by_storage(h->cfg, [&](auto tag) {
-        for (int s = 0; s < nsteps; ++s) one_step<decltype(tag)>(*h, nullptr, nullptr, s == 0);
+        for (int s = 0; s < nsteps;) s += one_launch<decltype(tag)>(*h, nsteps - s, nullptr, nullptr, s == 0);
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? 0 : fail(BGK_EHIP, "step launch: %s", hipGetErrorString(e));
     });
@@ -585,9 +523,11 @@ int bgk_time_steps(bgk_handle* h, int nsteps, double* total_ms, double* collide_
     ENG_HIP(hipStreamSynchronize(h->stream));
     hipEvent_t e0 = h->events[0], e1 = h->events[1];
     ENG_HIP(hipEventRecord(e0, h->stream));
+    int launches = 0;
     int rc = by_storage(h->cfg, [&](auto tag) {
-        for (int s = 0; s < nsteps; ++s)
-            one_step<decltype(tag)>(*h, h->events[2 + 2 * s], h->events[3 + 2 * s], s == 0);
+        for (int s = 0; s < nsteps; ++launches)
+            s += one_launch<decltype(tag)>(*h, nsteps - s, h->events[2 + 2 * launches], h->events[3 + 2 * launches],
+                                           s == 0);
         return 0;
     });
     if (rc) return rc;
@@ -596,7 +536,7 @@ int bgk_time_steps(bgk_handle* h, int nsteps, double* total_ms, double* collide_
     float ms = 0;
     ENG_HIP(hipEventElapsedTime(&ms, e0, e1));
     double ksum = 0;
-    for (int s = 0; s < nsteps; ++s) {
+    for (int s = 0; s < launches; ++s) {
         float k = 0;
         ENG_HIP(hipEventElapsedTime(&k, h->events[2 + 2 * s], h->events[3 + 2 * s]));
         ksum += k;

@@ -5,6 +5,7 @@
 
 #include "../../include/bgk3d_engine.h"
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -12,6 +13,7 @@
 #include "collide.hpp"
 #include "common.hpp"
 #include "d3q19.hpp"
+#include "pair.hpp"
 #include "reduce.hpp"
 #include "storage.hpp"
 #include "v1_kernels.hpp"
@@ -23,8 +25,9 @@ struct bgk_handle {
     // Layout of a lattice: the population planes of one z level lie next to
     // each other, population d of cell (i,j,k) at
     //   mem[buf] + base + d*plane + i + nx*j + nxy*k,
-    // plane = nx*ny, z stride nxy = 19*plane (lattice 1 holds 18 populations
-    // and leaves the 19th slot unused).  Rows are padded to whole 128-byte
+    // plane = nx*ny, z stride nxy = 19*plane.  Direction 19 is in lattice
+    // `rest`: single steps update it in place, pairs of steps move it to the
+    // other lattice's slot.  Rows are padded to whole 128-byte
     // lines and base puts i = 1 on a line start.  A wave's 19 loads and 19
     // stores then fall in two windows of 19 planes instead of 37 arrays
     // scattered over the whole region: fewer DRAM pages and translation
@@ -34,9 +37,12 @@ struct bgk_handle {
     // compact layout: rows of l + 2 cells (collide_compact), else rows padded
     // to whole lines (collide_fused)
     bool compact = false;
+    // two steps per launch (collide_pair) where two are left, in tiles pgrid
+    bool pair = false;
+    bgk::PairGrid pgrid{};
     void* mem[2] = {nullptr, nullptr};
     size_t bytes = 0;
-    int cur = 0;
+    int cur = 0, rest = 0;
     hipStream_t stream = nullptr;
     double omega = 0, fgrad = 0, lidforce = 0, u_inflow = 0, cte_s = 0;
     // obstacle
@@ -60,7 +66,7 @@ struct bgk_handle {
     template <typename S>
     S* cur_a(int d) const
     {
-        return d == 18 ? arr<S>(0, 18) : arr<S>(cur, d);
+        return arr<S>(d == 18 ? rest : cur, d);
     }
     template <typename S>
     bgk::Lattice19<S> current() const
@@ -139,6 +145,31 @@ int by_storage(const bgk_config& c, F&& f)
 // The collision runs in FP64 (DOUBLE_P storage, or the MIXED2 form).
 inline bool compute_double(const bgk_config& c) { return c.storage == BGK_F64 || c.mixed == 2; }
 
+// Tiles of the two-step kernel for this configuration, if two steps per
+// launch are faster than two launches of one.  Estimates in us from measured
+// launches: a single step takes 1.5 + its bytes at 6.2 TB/s, at least 4.6; a
+// pair 2.5 + its cost (pair_grid) times 0.42 in FP32 (0.38 ... 0.43 over
+// cavities, Taylor-Green, channel and the sphere, 64^3 ... 900 x 150^2), 0.48
+// in MIXED2 and 0.80 in FP64.  Measured per step, one step a launch against
+// two: FP32 256^3 410 / 268, 192^3 175 / 112, 64^3 9.7 / 6.3, FP64 192^3 359 /
+// 227.  LES with FP64 arithmetic stays with one (152 against 143 at 201 x 135
+// x 99: more values live than registers), 16-bit storage too (118 against 108
+// for the FP16 channel at 512 x 128^2: bound by issue, half the bytes).
+inline bool prefer_pair(const bgk_config& c, long plane, PairGrid& g)
+{
+    const size_t es = storage_bytes(c.storage);
+    const bool wide = compute_double(c);
+    if (es < 4 || c.layout == 2 || (c.les && wide)) return false;
+    // a lane's 32-bit byte offset spans up to four z levels (pair_tile)
+    if (80.0 * (double)es * (double)plane >= 4.0e9) return false;
+    double cost;
+    const int rows = es == 8 ? PairShape<double>::TY : (wide ? PairShape<mix32_t>::TY : PairShape<float>::TY);
+    g = pair_grid(c.l, c.m, c.n, rows, cost);
+    const double cells = (double)c.l * c.m * c.n;
+    const double two = 2 * std::max(4.6, 1.5 + 38.0 * (double)es * cells / 6.2e6);
+    return 2.5 + cost * (es == 8 ? 0.80 : (wide ? 0.48 : 0.42)) < two;
+}
+
 // Validate `c` and fill the layout and the derived parameters of `h`
 // (no device call, no allocation).
 int handle_setup(bgk_handle& h, const bgk_config& c);
@@ -161,13 +192,15 @@ __host__ __device__ inline uint32_t step_seed(uint32_t cfg_seed, long long steps
     return hash32(cfg_seed ^ hash32((uint32_t)steps * 0x9e3779b9U + 1u));
 }
 
-// Arguments of the fused kernel for the step that reads lattice `cur`.
+// Arguments of the fused kernel for the step that reads lattice `cur` and
+// finds direction 19 in lattice `rest`.
 template <typename S>
-FusedArgs<S> fused_args(const bgk_handle& h, int cur)
+FusedArgs<S> fused_args(const bgk_handle& h, int cur, int rest)
 {
     typedef typename Storage<S>::compute C;
     FusedArgs<S> p{};
-    for (int d = 0; d < 19; ++d) p.a[d] = d == 18 ? h.arr<S>(0, 18) : h.arr<S>(cur, d);
+    for (int d = 0; d < 19; ++d) p.a[d] = h.arr<S>(d == 18 ? rest : cur, d);
+    p.brest = h.arr<S>(1 - rest, 18);
     for (int d = 0; d < 18; ++d) p.b[d] = h.arr<S>(1 - cur, d);
     p.l = h.cfg.l;
     p.m = h.cfg.m;
@@ -196,10 +229,16 @@ FusedArgs<S> fused_args(const bgk_handle& h, int cur)
     else
         p.lend = h.cfg.boundary == BGK_BC_INFLOW ? 0 : (int)round_up(h.cfg.l, h.A);
     p.seed = step_seed(h.cfg.seed, h.steps);
+    p.seed2 = step_seed(h.cfg.seed, h.steps + 1);
     p.pstride = h.plane;
     p.uin = (C)h.u_inflow;
     return p;
 }
+
+// Queue the collide of the next step, or of the next two in one launch
+// (launch.hpp).
+template <typename S>
+void launch_step(bgk_handle& h, bool pair);
 
 }  // namespace eng
 }  // namespace bgk

@@ -72,21 +72,23 @@ constexpr int kMaxSkips = 8;
 
 template <typename S>
 struct BatchSlot {
-    FusedArgs<S> args[2];  // indexed by the lattice the step reads
+    FusedArgs<S> args[2];  // of the chunk's even and odd launches (each launch swaps the lattices)
     RowMap rm;
+    PairGrid pg;           // tiles (two steps per launch)
     int gy;                // row blocks along j (padded rows)
     int nbx;               // position blocks per plane (compact rows)
-    int par0;              // lattice read at chunk step 0
     uint32_t cfg_seed;
     long long steps0;      // steps completed before the chunk
     uint32_t block0;       // first block of this request in the launch
+    uint32_t tile0;        // first tile of this request in a two-step launch
 };
 
 // One time step of every request of one storage group.  The lid-driven
 // cavity: bounce-back walls in x and y, lid at z = n + 1 (SRC/bcond.driven.F90).
 template <typename S, int SR>
 __global__ __launch_bounds__(64 * kServeWaves) __attribute__((amdgpu_waves_per_eu(FusedWaves<S, 0>::value))) void
-collide_batched(const BatchSlot<S>* __restrict__ slots, const uint32_t* __restrict__ owner, uint32_t base, int t)
+collide_batched(const BatchSlot<S>* __restrict__ slots, const uint32_t* __restrict__ owner, uint32_t base, int t,
+                int launch)
 {
     const uint32_t b = base + blockIdx.x;
     const BatchSlot<S>& sl = slots[owner[b]];
@@ -97,7 +99,7 @@ collide_batched(const BatchSlot<S>* __restrict__ slots, const uint32_t* __restri
     const int by = (int)(rest % (uint32_t)sl.gy);
     const int bz = (int)(rest / (uint32_t)sl.gy);
     const uint32_t seed = SR ? step_seed(sl.cfg_seed, sl.steps0 + t) : 0u;
-    fused_rows<S, AX_WALL, AX_WALL, AX_LID, false, 0, SR>(sl.args[(sl.par0 + t) & 1], rm, bx, by, bz, seed);
+    fused_rows<S, AX_WALL, AX_WALL, AX_LID, false, 0, SR>(sl.args[launch & 1], rm, bx, by, bz, seed);
 }
 
 // The same for requests in the compact layout (collide_compact's mapping,
@@ -105,7 +107,7 @@ collide_batched(const BatchSlot<S>* __restrict__ slots, const uint32_t* __restri
 template <typename S, int SR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FusedWaves<S, 0>::value))) void
 collide_batched_compact(const BatchSlot<S>* __restrict__ slots, const uint32_t* __restrict__ owner, uint32_t base,
-                        int t)
+                        int t, int launch)
 {
     const uint32_t b = base + blockIdx.x;
     const BatchSlot<S>& sl = slots[owner[b]];
@@ -113,7 +115,20 @@ collide_batched_compact(const BatchSlot<S>* __restrict__ slots, const uint32_t* 
     const int bx = (int)(lb % (uint32_t)sl.nbx);
     const int bz = (int)(lb / (uint32_t)sl.nbx);
     const uint32_t seed = SR ? step_seed(sl.cfg_seed, sl.steps0 + t) : 0u;
-    compact_cells<S, AX_WALL, AX_WALL, AX_LID, false, 0, SR>(sl.args[(sl.par0 + t) & 1], bx, bz, seed);
+    compact_cells<S, AX_WALL, AX_WALL, AX_LID, false, 0, SR>(sl.args[launch & 1], bx, bz, seed);
+}
+
+// Two steps of every request of a sub-batch (collide_pair's tiles): the n
+// tiles from `base` on, owner[] the request of each.
+template <typename S>
+__global__ __launch_bounds__(64 * (PairShape<S>::TY + 3)) void collide_pair_batched(
+    const BatchSlot<S>* __restrict__ slots, const uint32_t* __restrict__ owner, uint32_t base, int n, int launch)
+{
+    const int b = xcd_tile((int)blockIdx.x, n);
+    if (b >= n) return;
+    const uint32_t tile = base + (uint32_t)b;
+    const BatchSlot<S>& sl = slots[__builtin_amdgcn_readfirstlane((int)owner[tile])];
+    pair_tile<S, AX_WALL, AX_WALL, AX_LID, false, 0, 0>(sl.args[launch & 1], sl.pg, (int)(tile - sl.tile0), 0u, 0u);
 }
 
 double clock_now()
@@ -184,13 +199,14 @@ struct Instance {
 };
 
 // Launch group of a request: storage type and rounding (which select the
-// kernel's template), plus 8 for the compact layout.
-int group_of(int storage, int rounding, bool compact)
+// kernel's template), plus 8 for the compact layout or 16 for two steps per
+// launch (padded rows).
+int group_of(const bgk_handle& h)
 {
-    const bool sr = rounding && (storage == BGK_F16 || storage == BGK_BF16);
-    return storage * 2 + (sr ? 1 : 0) + (compact ? 8 : 0);
+    const bool sr = h.cfg.rounding && (h.cfg.storage == BGK_F16 || h.cfg.storage == BGK_BF16);
+    return h.cfg.storage * 2 + (sr ? 1 : 0) + (h.compact ? 8 : 0) + (h.pair ? 16 : 0);
 }
-constexpr int kGroups = 16;
+constexpr int kGroups = 24;
 
 bgk_config request_config(const bgks_request& r, int device)
 {
@@ -229,7 +245,7 @@ struct bgks_server {
     // per storage group: device tables and pinned staging
     struct Group {
         void* d_slots = nullptr;
-        uint32_t* d_owner = nullptr;
+        uint32_t* d_owner = nullptr;  // of every block, then of every tile (two-step launches)
         void* h_slots = nullptr;
         uint32_t* h_owner = nullptr;
         size_t slot_bytes_cap = 0, owner_cap = 0;
@@ -268,7 +284,8 @@ int grow_group(bgks_server& s, bgks_server::Group& g, size_t slot_bytes, size_t 
 // step count at the chunk start) and the owner of every block.
 struct SubBatch {
     uint32_t block0, nblocks;
-    int single;  // the member that is alone in this sub-batch, else -1
+    uint32_t tile0, ntiles;  // two-step launches
+    int single;              // the member that is alone in this sub-batch, else -1
 };
 
 template <typename S>
@@ -276,26 +293,28 @@ int prepare_group(bgks_server& s, bgks_server::Group& g, const std::vector<Insta
                   std::vector<SubBatch>& subs, hipStream_t stream)
 {
     std::vector<BatchSlot<S>> slots(members.size());
-    uint32_t total = 0;
+    std::vector<size_t> sub_of(members.size());
+    uint32_t total = 0, tiles = 0;
     size_t sub_bytes = 0;
     subs.clear();
+    const bool pair = !members.empty() && members[0]->h.pair;
     for (size_t q = 0; q < members.size(); ++q) {
         bgk_handle& h = members[q]->h;
         if (subs.empty() || (sub_bytes > 0 && sub_bytes + members[q]->len > kSubBatchBytes)) {
-            subs.push_back({total, 0, (int)q});
+            subs.push_back({total, 0, 0, 0, (int)q});
             sub_bytes = 0;
         } else {
             subs.back().single = -1;
         }
         sub_bytes += members[q]->len;
+        sub_of[q] = subs.size() - 1;
         BatchSlot<S>& sl = slots[q];
-        sl.args[0] = fused_args<S>(h, 0);
-        sl.args[1] = fused_args<S>(h, 1);
+        sl.args[0] = fused_args<S>(h, h.cur, h.rest);
+        sl.args[1] = fused_args<S>(h, 1 - h.cur, pair ? 1 - h.rest : h.rest);
         sl.args[0].bad = sl.args[1].bad = s.d_flags + members[q]->flag;
         sl.rm = row_map_capped(h.cfg.l, kServeWaves);
         sl.gy = ceil_div(h.cfg.m, sl.rm.rpb);
         sl.nbx = ceil_div(sl.args[0].lend, 256);
-        sl.par0 = h.cur;
         sl.cfg_seed = h.cfg.seed;
         sl.steps0 = h.steps;
         sl.block0 = total;
@@ -306,27 +325,62 @@ int prepare_group(bgks_server& s, bgks_server::Group& g, const std::vector<Insta
         total += (uint32_t)nb;
         subs.back().nblocks += (uint32_t)nb;
     }
-    if (int rc = grow_group(s, g, slots.size() * sizeof(BatchSlot<S>), total)) return rc;
-    std::memcpy(g.h_slots, slots.data(), slots.size() * sizeof(BatchSlot<S>));
+    if (pair) {
+        // A request in company gets tiles for the share of the CUs that its
+        // cells are of its sub-batch's.
+        std::vector<double> cells(subs.size(), 0.0);
+        auto count = [](const bgk_config& c) { return (double)c.l * c.m * c.n; };
+        for (size_t q = 0; q < members.size(); ++q) cells[sub_of[q]] += count(members[q]->h.cfg);
+        for (size_t q = 0; q < members.size(); ++q) {
+            const bgk_config& c = members[q]->h.cfg;
+            SubBatch& sb = subs[sub_of[q]];
+            PairGrid& pg = slots[q].pg;
+            double cost;
+            pg = members[q]->h.pgrid;
+            if (sb.single < 0)
+                pg = pair_grid(c.l, c.m, c.n, PairShape<S>::TY, cost,
+                               std::max(1.0, 256 * count(c) / cells[sub_of[q]]));
+            if (sb.ntiles == 0) sb.tile0 = tiles;
+            slots[q].tile0 = tiles;
+            tiles += (uint32_t)pg.total;
+            sb.ntiles += (uint32_t)pg.total;
+        }
+    }
+    if (int rc = grow_group(s, g, slots.size() * sizeof(BatchSlot<S>), (size_t)total + tiles)) return rc;
     for (size_t q = 0; q < members.size(); ++q) {
         const uint32_t b0 = slots[q].block0;
         const uint32_t b1 = q + 1 < members.size() ? slots[q + 1].block0 : total;
         std::fill(g.h_owner + b0, g.h_owner + b1, (uint32_t)q);
+        slots[q].tile0 += total;  // the tiles' owners follow the blocks'
+        std::fill_n(g.h_owner + slots[q].tile0, slots[q].pg.total, (uint32_t)q);
     }
+    for (SubBatch& sb : subs) sb.tile0 += total;
+    std::memcpy(g.h_slots, slots.data(), slots.size() * sizeof(BatchSlot<S>));
     ENG_HIP(hipMemcpyAsync(g.d_slots, g.h_slots, slots.size() * sizeof(BatchSlot<S>), hipMemcpyHostToDevice,
                            stream));
-    ENG_HIP(hipMemcpyAsync(g.d_owner, g.h_owner, (size_t)total * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
+    ENG_HIP(hipMemcpyAsync(g.d_owner, g.h_owner, ((size_t)total + tiles) * sizeof(uint32_t),
+                           hipMemcpyHostToDevice, stream));
     return 0;
 }
 
+// Queue the launch number `launch` of a chunk for one sub-batch, of the steps
+// from chunk step t on: two with `pair`, else one.
 template <typename S, int SR>
-void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, hipStream_t stream, bool compact)
+void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, int launch, bool pair, hipStream_t stream,
+                  bool compact)
 {
+    const BatchSlot<S>* d_slots = static_cast<const BatchSlot<S>*>(g.d_slots);
     if (sb.single >= 0) {
         // the engine's launch for a driven cavity (engine.hip launch_fused)
         const BatchSlot<S>& sl = static_cast<const BatchSlot<S>*>(g.h_slots)[sb.single];
-        FusedArgs<S> p = sl.args[(sl.par0 + t) & 1];
+        FusedArgs<S> p = sl.args[launch & 1];
         p.seed = step_seed(sl.cfg_seed, sl.steps0 + t);
+        if constexpr (kPairs<S, 0>) {
+            if (pair) {
+                launch_pair<S, AX_WALL, AX_WALL, AX_LID, false, 0, SR>(p, sl.pg, stream);
+                return;
+            }
+        }
         if (compact) {
             hipLaunchKernelGGL((collide_compact<S, AX_WALL, AX_WALL, AX_LID, false, 0, SR>),
                                dim3((unsigned)ceil_div(p.lend, 256), (unsigned)p.n), dim3(256), compact_lds_cap<S>(),
@@ -345,12 +399,20 @@ void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, hipStream_t 
                            fused_block(rm), 0, stream, p, rm);
         return;
     }
+    if constexpr (kPairs<S, 0>) {
+        if (pair) {
+            hipLaunchKernelGGL((collide_pair_batched<S>), dim3((unsigned)pair_blocks((int)sb.ntiles)),
+                               dim3(64 * (PairShape<S>::TY + 3)), 0, stream, d_slots, g.d_owner, sb.tile0,
+                               (int)sb.ntiles, launch);
+            return;
+        }
+    }
     if (compact)
         hipLaunchKernelGGL((collide_batched_compact<S, SR>), dim3(sb.nblocks), dim3(256), compact_lds_cap<S>(), stream,
-                           static_cast<const BatchSlot<S>*>(g.d_slots), g.d_owner, sb.block0, t);
+                           d_slots, g.d_owner, sb.block0, t, launch);
     else
-        hipLaunchKernelGGL((collide_batched<S, SR>), dim3(sb.nblocks), dim3(64 * kServeWaves), 0, stream,
-                           static_cast<const BatchSlot<S>*>(g.d_slots), g.d_owner, sb.block0, t);
+        hipLaunchKernelGGL((collide_batched<S, SR>), dim3(sb.nblocks), dim3(64 * kServeWaves), 0, stream, d_slots,
+                           g.d_owner, sb.block0, t, launch);
 }
 
 template <typename F>
@@ -639,13 +701,19 @@ int bgks_advance(bgks_server* s, long long* done_ids, int max_done, int* n_done)
         const double per_step_ms = s->ns_per_cell_step * (double)cells_in_flight * 1e-6;
         K = std::min(K, std::max(1LL, (long long)(s->chunk_ms / per_step_ms)));
     }
+    // an even chunk leaves no single step to requests that take two per launch
+    const bool pairs = std::any_of(active.begin(), active.end(), [](const Instance* in) { return in->h.pair; });
+    if (pairs && K > 1 && std::all_of(active.begin(), active.end(), [&](const Instance* in) {
+            return in->req.steps - in->h.steps > K;
+        }))
+        K &= ~1LL;
     K = std::max(K, 0LL);
 
     bool ran = false;
     if (K > 0 && !active.empty()) {
         std::vector<Instance*> members[kGroups];
         for (Instance* in : active)
-            members[group_of(in->h.cfg.storage, in->h.cfg.rounding, in->h.compact)].push_back(in);
+            members[group_of(in->h)].push_back(in);
         std::vector<SubBatch> subs[kGroups];
         for (int g = 0; g < kGroups; ++g) {
             if (members[g].empty()) continue;
@@ -660,22 +728,29 @@ int bgks_advance(bgks_server* s, long long* done_ids, int max_done, int* n_done)
         // sub-batches streaming side by side on a second stream ran the mix
         // about 6 % slower than one after the other.
         for (int g = 0; g < kGroups; ++g)
-            for (const SubBatch& sb : subs[g])
-                for (long long t = 0; t < K; ++t) {
+            for (const SubBatch& sb : subs[g]) {
+                int launch = 0;
+                for (long long t = 0; t < K; ++launch) {
+                    const bool pair = (g & 16) != 0 && K - t >= 2;
                     by_group(g, [&](auto tag, auto sr) {
-                        launch_group<decltype(tag), decltype(sr)::value>(s->groups[g], sb, (int)t, s->stream,
-                                                                          g >= 8);
+                        launch_group<decltype(tag), decltype(sr)::value>(s->groups[g], sb, (int)t, launch, pair,
+                                                                          s->stream, (g & 8) != 0);
                         return 0;
                     });
+                    t += pair ? 2 : 1;
                     ++s->launches;
                 }
+            }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return fail(BGK_EHIP, "batched step launch: %s", hipGetErrorString(e));
         ENG_HIP(hipStreamSynchronize(s->stream));
         s->ns_per_cell_step = (clock_now() - t0) * 1e9 / ((double)K * (double)cells_in_flight);
         for (Instance* in : active) {
             in->h.steps += K;
-            in->h.cur = (int)((in->h.cur + K) & 1);
+            // every launch swaps the lattices, a two-step launch direction 19's too
+            const long long pairs = in->h.pair ? K / 2 : 0;
+            in->h.cur = (int)((in->h.cur + K - pairs) & 1);
+            in->h.rest = (int)((in->h.rest + pairs) & 1);
             s->cell_steps += (long long)in->h.cfg.l * in->h.cfg.m * in->h.cfg.n * K;
         }
         ++s->chunks;

@@ -1,0 +1,68 @@
+"""Two steps per launch (handle API, collide_pair): the same bits as the oracle
+and as single steps, at the edges of its tiles.
+
+Tiles are 64 cells in x and up to 13 rows (8 or 9 with FP64 arithmetic), cut
+into ranges of planes; the sizes below leave one cell, one row or one plane
+over, fit exactly, or are smaller than a tile's border.
+"""
+import numpy as np
+import pytest
+
+import oracle_support as O
+from bgk3d_gpu_amd.cases import Case
+from bgk3d_gpu_amd.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1, 1), (2, 2, 2), (63, 1, 2), (64, 13, 3), (65, 14, 1), (66, 27, 5), (128, 8, 9), (129, 9, 4)]
+CASES = {
+    "ldc": dict(boundary="ldc", svisc=0.05, u0=0.1),
+    "periodic": dict(boundary="periodic", svisc=0.02, u0=0.05, init=1),
+    "channel": dict(boundary="channel", svisc=0.1, u0=0.5),
+    "inflow": dict(boundary="inflow", svisc=0.05, u0=0.1),
+    "ldc_les": dict(boundary="ldc", svisc=0.01, u0=0.1, les=True),
+}
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+@pytest.mark.parametrize("name", list(CASES))
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
+def test_pairs_match_oracle(gpu, size, name, storage):
+    """Six steps in one call (three launches) and in calls of 1, 2 and 3."""
+    case = Case(l=size[0], m=size[1], n=size[2], **CASES[name])
+    print(f"[gpu] pairs {name} {storage} {size}", flush=True)
+    out = []
+    for chunks in ((6,), (1, 2, 3)):
+        with Engine(case, storage, layout=1) as eng:
+            for c in chunks:
+                eng.step(c)
+            out.append(eng.populations())
+    prec = "sp" if storage == "f32" else "dp"
+    A = O.new_lattice(case.l, case.m, case.n, prec)
+    B = O.new_lattice(case.l, case.m, case.n, prec)
+    O.init(A, case.l, case.m, case.n, prec, mode=case.init, u00=case.u00)
+    O.run(case.boundary, A, B, case.l, case.m, case.n, 6, prec=prec, svisc=case.svisc, u0=case.u0, les=case.les,
+          cte_s=case.cte_s)
+    ref = A[:, 1:-1, 1:-1, 1:-1].astype(np.float64)
+    assert np.array_equal(out[0], ref), f"max |diff| {np.abs(out[0] - ref).max()}"
+    assert np.array_equal(out[1], ref)
+
+
+@pytest.mark.parametrize("storage,mixed", [("f32", 0), ("f64", 0), ("f32", 2)])
+@pytest.mark.parametrize("kw", [dict(boundary="periodic", init=1, obstacle=True), dict(boundary="inflow", obstacle=True),
+                                dict(boundary="channel", wall_axis=2), dict(boundary="channel", wall_axis=2, force_axis=3),
+                                dict(boundary="channel", force_axis=2), dict(boundary="ldc")],
+                         ids=["periodic-obstacle", "inflow-obstacle", "walls-y", "walls-y-force-z", "force-y", "ldc"])
+def test_pairs_match_single_steps(gpu, kw, storage, mixed):
+    """Forms the oracle's runs above leave out, against step(1) calls: links of
+    an obstacle that spans several tiles, walls in y with z periodic, MIXED2."""
+    case = Case(l=70, m=30, n=24, svisc=0.03, u0=0.1, **kw)
+    print(f"[gpu] pairs against singles {kw} {storage} mixed={mixed}", flush=True)
+    out = []
+    for chunks in ((20,), (1,) * 20):
+        with Engine(case, storage, layout=1, mixed=mixed) as eng:
+            for c in chunks:
+                eng.step(c)
+            out.append(eng.populations())
+    assert np.isfinite(out[0]).all() and np.any(out[0] != 0)
+    assert np.array_equal(out[0], out[1])
