@@ -550,18 +550,15 @@ int bgk_diagno(bgk_handle* h, double out[5])
 {
     if (!h || !out) return fail(BGK_EINVAL, "bad arguments");
     ENG_HIP(hipSetDevice(h->cfg.device));
-    const long rows = (long)h->cfg.m * h->cfg.n;
-    const int nb = (int)std::min<long>(rows, kRedBlocks);
+    const int nb = diagno_blocks((long)h->cfg.m * h->cfg.n);
     int rc = by_storage(h->cfg, [&](auto tag) {
         typedef decltype(tag) S;
         hipLaunchKernelGGL(diagno_partial<S>, dim3(nb), dim3(kRedThreads), 0, h->stream, h->current<S>(), h->geom(),
-                           cte_one<S>(), h->scratch + 5);
-        hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, h->stream, h->scratch + 5, nb,
-                           h->scratch);
+                           cte_one<S>(), h->scratch);
+        hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, h->stream, h->scratch, nb, h->hscratch);
         return 0;
     });
     if (rc) return rc;
-    ENG_HIP(hipMemcpyAsync(h->hscratch, h->scratch, 5 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     ENG_HIP(hipStreamSynchronize(h->stream));
     const double fl = (double)(float)h->cfg.l, fm = (double)(float)h->cfg.m, fn = (double)(float)h->cfg.n;
     for (int q = 0; q < 5; ++q) out[q] = (h->hscratch[q] / fl) / fm / fn;
@@ -584,12 +581,10 @@ int bgk_draglift(bgk_handle* h, double out[3])
         typedef decltype(tag) S;
         hipLaunchKernelGGL(draglift_box<S>, dim3(nb), dim3(kRedThreads), 0, h->stream, h->current<S>(), h->geom(),
                            h->omask, h->mk[0], h->mk[1], h->mk[2], h->mk[3], h->mk[4], h->mk[5], is, ie, js, je, ks,
-                           ke, h->scratch + 5);
-        hipLaunchKernelGGL(fold_partials<3>, dim3(1), dim3(kRedThreads), 0, h->stream, h->scratch + 5, nb,
-                           h->scratch);
+                           ke, h->scratch);
+        hipLaunchKernelGGL(fold_partials<3>, dim3(1), dim3(kRedThreads), 0, h->stream, h->scratch, nb, h->hscratch);
         return 0;
     });
-    ENG_HIP(hipMemcpyAsync(h->hscratch, h->scratch, 3 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     ENG_HIP(hipStreamSynchronize(h->stream));
     // norm = uno/(u_inflow*u_inflow*radius) in the working kind (SRC/draglift.F90:178)
     double norm;

@@ -52,6 +52,8 @@ __device__ __forceinline__ void block_sum(double (&v)[NV])
 }
 
 // Second pass: one block folds nblk partials (layout [blk][NV]) in order.
+// `out` is host memory the GPU can write (hipHostMalloc): the totals are there
+// when the stream has been waited for, without a copy of their own.
 template <int NV>
 __global__ __launch_bounds__(kRedThreads) void fold_partials(const double* __restrict__ part, int nblk,
                                                              double* __restrict__ out)
@@ -70,9 +72,26 @@ __global__ __launch_bounds__(kRedThreads) void fold_partials(const double* __res
     }
 }
 
+// Blocks of diagno_partial: a wave per row of cells, at most kRedBlocks
+// blocks of four waves (then a wave takes several rows).
+inline int diagno_blocks(long rows) { return (int)((rows + 3) / 4 < kRedBlocks ? (rows + 3) / 4 : kRedBlocks); }
+
+// The 19 stored values of cell s.
+template <typename S>
+__device__ __forceinline__ void load_cell(const Lattice19<S>& a, long s, typename Storage<S>::compute (&x)[19])
+{
+#pragma unroll
+    for (int d = 0; d < 19; ++d) x[d] = Storage<S>::load(a.p[d] + s);
+}
+
 // diagno (SRC/diagno.F90:89-131): per interior cell rho, u, v, w and
 // 0.5|u|^2 in the storage kind; partial sums {u, v, w, rho, ke} in FP64.
-// Rows (j,k) are distributed over blocks; lanes walk i.
+// A wave takes a row (j, k) at a time, its lanes walk i: rows shorter than a
+// block's 256 threads leave none of them idle.  With varm below (one read of
+// the lattice instead of two, by all CUs) and the results of every diagnostic
+// written to host memory by its last kernel, the set printed at a check
+// (means, plane means, three lines, a probe, drag) took 410 us at 450 x 150 x
+// 150 FP32 instead of 815.
 template <typename S>
 __global__ __launch_bounds__(kRedThreads) void diagno_partial(Lattice19<S> a, Geometry g,
                                                               typename Storage<S>::compute cte1,
@@ -81,13 +100,12 @@ __global__ __launch_bounds__(kRedThreads) void diagno_partial(Lattice19<S> a, Ge
     typedef typename Storage<S>::compute R;
     double v[5] = {0, 0, 0, 0, 0};
     const long rows = (long)g.m * g.n;
-    for (long r = blockIdx.x; r < rows; r += gridDim.x) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (long r = (long)blockIdx.x * 4 + wave; r < rows; r += (long)gridDim.x * 4) {
         const int j = 1 + (int)(r % g.m), k = 1 + (int)(r / g.m);
-        for (int i = 1 + threadIdx.x; i <= g.l; i += kRedThreads) {
-            const long s = gidx(g, i, j, k);
+        for (int i = 1 + lane; i <= g.l; i += 64) {
             R x[19];
-#pragma unroll
-            for (int d = 0; d < 19; ++d) x[d] = Storage<S>::load(a.p[d] + s);
+            load_cell(a, gidx(g, i, j, k), x);
             const R rho = density_ref(x, cte1);
             const R rhoinv = R(1) / rho;
             const R xj = (x[0] + x[1] + x[2] + x[3] + x[4] - x[9] - x[10] - x[11] - x[12] - x[13]) * rhoinv;
@@ -107,56 +125,64 @@ __global__ __launch_bounds__(kRedThreads) void diagno_partial(Lattice19<S> a, Ge
     }
 }
 
-// varm (SRC/varm.F90:56-92): velocity sums per z-plane k (block = plane)
-// -> out[3*(k-1) + {0,1,2}] = {u, w(y-vel), v(z-vel)}.
+// varm (SRC/varm.F90:56-92), first pass: the sums of u, w (y velocity), v (z
+// velocity) and the density over each row (j, k), part[4 * row + {0,1,2,3}],
+// row = (j - 1) + m (k - 1).  A wave per row, so the lattice is read once with
+// the whole GPU at work (a block per plane left 106 of 256 CUs idle at 150
+// planes, and the planes along j were a second read).
 template <typename S>
-__global__ __launch_bounds__(kRedThreads) void varm_planes_k(Lattice19<S> a, Geometry g,
-                                                             typename Storage<S>::compute cte1,
-                                                             double* __restrict__ out)
+__global__ __launch_bounds__(kRedThreads) void varm_rows(Lattice19<S> a, Geometry g, typename Storage<S>::compute cte1,
+                                                         double* __restrict__ part)
 {
     typedef typename Storage<S>::compute R;
-    const int k = 1 + blockIdx.x;
-    double v[3] = {0, 0, 0};
-    const long cells = (long)g.l * g.m;
-    for (long c = threadIdx.x; c < cells; c += kRedThreads) {
-        const int i = 1 + (int)(c % g.l), j = 1 + (int)(c / g.l);
-        const long s = gidx(g, i, j, k);
+    const int lane = threadIdx.x & 63;
+    const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= (long)g.m * g.n) return;
+    const int j = 1 + (int)(r % g.m), k = 1 + (int)(r / g.m);
+    double v[4] = {0, 0, 0, 0};
+    for (int i = 1 + lane; i <= g.l; i += 64) {
         R x[19];
-#pragma unroll
-        for (int d = 0; d < 19; ++d) x[d] = Storage<S>::load(a.p[d] + s);
-        const R rhoinv = R(1) / density_ref(x, cte1);
+        load_cell(a, gidx(g, i, j, k), x);
+        const R rho = density_ref(x, cte1);
+        const R rhoinv = R(1) / rho;
         v[0] += (double)((x[0] + x[1] + x[2] + x[3] + x[4] - x[9] - x[10] - x[11] - x[12] - x[13]) * rhoinv);
         v[1] += (double)((x[2] + x[6] + x[7] + x[8] + x[11] - x[0] - x[9] - x[15] - x[16] - x[17]) * rhoinv);
         v[2] += (double)((x[3] + x[5] + x[6] + x[12] + x[17] - x[1] - x[8] - x[10] - x[14] - x[15]) * rhoinv);
+        v[3] += (double)rho;
     }
-    block_sum<3>(v);
-    if (threadIdx.x == 0) {
-        out[3 * (k - 1) + 0] = v[0];
-        out[3 * (k - 1) + 1] = v[1];
-        out[3 * (k - 1) + 2] = v[2];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = wave_sum(v[q]);
+    if (lane == 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) part[4 * r + q] = v[q];
     }
 }
 
-// varm density sums per y-plane j (block = plane) -> out[j-1].
-template <typename S>
-__global__ __launch_bounds__(kRedThreads) void varm_planes_j(Lattice19<S> a, Geometry g,
-                                                             typename Storage<S>::compute cte1,
-                                                             double* __restrict__ out)
+// Second pass: blocks 0..n-1 fold the velocities of plane k = block + 1 into
+// out[3 * block + {0,1,2}], blocks n..n+m-1 the densities of plane j into
+// out[3 * n + block - n].  `out` as in fold_partials.
+static __global__ __launch_bounds__(kRedThreads) void varm_fold(const double* __restrict__ part, int m, int n,
+                                                         double* __restrict__ out)
 {
-    typedef typename Storage<S>::compute R;
-    const int j = 1 + blockIdx.x;
-    double v[1] = {0};
-    const long cells = (long)g.l * g.n;
-    for (long c = threadIdx.x; c < cells; c += kRedThreads) {
-        const int i = 1 + (int)(c % g.l), k = 1 + (int)(c / g.l);
-        const long s = gidx(g, i, j, k);
-        R x[19];
+    const int b = (int)blockIdx.x;
+    double v[3] = {0, 0, 0};
+    if (b < n) {
+        for (int j = threadIdx.x; j < m; j += kRedThreads) {
 #pragma unroll
-        for (int d = 0; d < 19; ++d) x[d] = Storage<S>::load(a.p[d] + s);
-        v[0] += (double)density_ref(x, cte1);
+            for (int q = 0; q < 3; ++q) v[q] += part[4 * ((long)b * m + j) + q];
+        }
+    } else {
+        for (int k = threadIdx.x; k < n; k += kRedThreads) v[0] += part[4 * ((long)k * m + (b - n)) + 3];
     }
-    block_sum<1>(v);
-    if (threadIdx.x == 0) out[j - 1] = v[0];
+    block_sum<3>(v);
+    if (threadIdx.x == 0) {
+        if (b < n) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) out[3 * b + q] = v[q];
+        } else {
+            out[3 * n + b - n] = v[0];
+        }
+    }
 }
 
 // draglift (SRC/draglift.F90:77-176): momentum exchange over fluid cells of

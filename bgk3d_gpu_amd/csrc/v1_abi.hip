@@ -22,8 +22,9 @@
 #include "../../include/bgk3d_gpu.h"
 
 #include <algorithm>
-#include <cstdlib>
 #include <cmath>
+#include <cstdlib>
+#include <cstring>
 
 #ifdef BGK_DOUBLE
 using real_t = double;
@@ -195,11 +196,12 @@ void launch_col(const Lattice19<real_t>& A, const Lattice19<real_t>& B, const Ge
 }
 
 // Cached scratch for the reductions (per device; single host thread, as in
-// the reference's driver).
+// the reference's driver): partial sums on the device, and pinned host memory
+// that the last kernel of a reduction writes its results to.
 struct Scratch {
     double* dev = nullptr;
     double* host = nullptr;
-    size_t cap = 0;
+    size_t dev_cap = 0, host_cap = 0;
 };
 
 Scratch& scratch_for_device()
@@ -210,21 +212,28 @@ Scratch& scratch_for_device()
     return s[dev & 63];
 }
 
-double* cached_scratch(size_t doubles, double** host)
+// At least dev_doubles on the device and host_doubles in pinned host memory;
+// false if either cannot be had.
+bool cached_scratch(size_t dev_doubles, size_t host_doubles, double** dev, double** host)
 {
     Scratch& s = scratch_for_device();
-    if (s.cap < doubles) {
+    if (s.dev_cap < dev_doubles) {
         if (s.dev) (void)hipFree(s.dev);
-        if (s.host) (void)hipHostFree(s.host);
         s.dev = nullptr;
-        s.host = nullptr;
-        s.cap = 0;
-        if (hipMalloc(&s.dev, doubles * sizeof(double)) != hipSuccess) return nullptr;
-        if (hipHostMalloc(&s.host, doubles * sizeof(double), hipHostMallocDefault) != hipSuccess) return nullptr;
-        s.cap = doubles;
+        s.dev_cap = 0;
+        if (hipMalloc(&s.dev, dev_doubles * sizeof(double)) != hipSuccess) return false;
+        s.dev_cap = dev_doubles;
     }
+    if (s.host_cap < host_doubles) {
+        if (s.host) (void)hipHostFree(s.host);
+        s.host = nullptr;
+        s.host_cap = 0;
+        if (hipHostMalloc(&s.host, host_doubles * sizeof(double), hipHostMallocDefault) != hipSuccess) return false;
+        s.host_cap = host_doubles;
+    }
+    *dev = s.dev;
     *host = s.host;
-    return s.dev;
+    return true;
 }
 
 // The device address of `scratch` on the current device, looked up once per
@@ -250,9 +259,9 @@ double* noalloc_scratch_ptr()
     return ptr[dev];
 }
 
-int fetch(const double* dev, double* host, size_t n)
+// Wait for the kernels that write a reduction's results to host memory.
+int finish()
 {
-    BGK_HIP_CHECK(hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, abi_stream()));
     BGK_HIP_CHECK(hipStreamSynchronize(abi_stream()));
     return 0;
 }
@@ -393,31 +402,33 @@ int bgk_set_stream(void* stream)
     return 0;
 }
 
+static void diagno_means(const double* sums, int l, int m, int n, double* out)
+{
+    // (x/float(l))/float(m)/float(n), SRC/diagno.F90:134-138
+    const double fl = (double)(float)l, fm = (double)(float)m, fn = (double)(float)n;
+    for (int q = 0; q < 5; ++q) out[q] = (sums[q] / fl) / fm / fn;
+}
+
 int diagno_gpu(real_t** a, int l, int m, int n, int nx, int ny, real_t cte1, double* out)
 {
     if (!shape_ok("diagno_gpu", l, m, n, nx, ny, a) || !out) return -1;
-    double* host = nullptr;
-    double* dev = cached_scratch((size_t)(kRedBlocks + 1) * 5, &host);
-    if (!dev) return -2;
-    const long rows = (long)m * n;
-    const int nb = (int)(rows < kRedBlocks ? rows : kRedBlocks);
+    double *dev = nullptr, *host = nullptr;
+    if (!cached_scratch((size_t)kRedBlocks * 5, 5, &dev, &host)) return -2;
+    const int nb = diagno_blocks((long)m * n);
     hipLaunchKernelGGL(diagno_partial<real_t>, dim3(nb), dim3(kRedThreads), 0, abi_stream(), lat_from(a),
-                       geom(l, m, n, nx, ny), cte1, dev + 5);
+                       geom(l, m, n, nx, ny), cte1, dev);
     report_launch("diagno_partial");
-    hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, abi_stream(), dev + 5, nb, dev);
+    hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, abi_stream(), dev, nb, host);
     report_launch("fold_partials");
-    if (int rc = fetch(dev, host, 5)) return rc;
-    // (x/float(l))/float(m)/float(n), SRC/diagno.F90:134-138
-    const double fl = (double)(float)l, fm = (double)(float)m, fn = (double)(float)n;
-    for (int q = 0; q < 5; ++q) out[q] = (host[q] / fl) / fm / fn;
+    if (int rc = finish()) return rc;
+    diagno_means(host, l, m, n, out);
     return 0;
 }
 
 int diagno_gpu_noalloc(real_t** a, int l, int m, int n, int nx, int ny, real_t cte1, double* out)
 {
     if (!shape_ok("diagno_gpu_noalloc", l, m, n, nx, ny, a) || !out) return -1;
-    const long rows = (long)m * n;
-    const int nb = (int)(rows < kRedBlocks ? rows : kRedBlocks);
+    const int nb = diagno_blocks((long)m * n);
     // the partials of nb blocks after the 5 totals
     if ((size_t)(nb + 1) * 5 > kNoAllocDoubles) {
         std::fprintf(stderr, "bgk3d_gpu: diagno_gpu_noalloc: %d partials exceed the static scratch of %zu doubles\n",
@@ -435,8 +446,7 @@ int diagno_gpu_noalloc(real_t** a, int l, int m, int n, int nx, int ny, real_t c
     double host[5];
     BGK_HIP_CHECK(hipMemcpyAsync(host, dev, sizeof host, hipMemcpyDeviceToHost, abi_stream()));
     BGK_HIP_CHECK(hipStreamSynchronize(abi_stream()));
-    const double fl = (double)(float)l, fm = (double)(float)m, fn = (double)(float)n;
-    for (int q = 0; q < 5; ++q) out[q] = (host[q] / fl) / fm / fn;
+    diagno_means(host, l, m, n, out);
     return 0;
 }
 
@@ -444,17 +454,15 @@ int varm_gpu(real_t** a, int l, int m, int n, int nx, int ny, real_t cte1, doubl
              double* den_j)
 {
     if (!shape_ok("varm_gpu", l, m, n, nx, ny, a) || !u_k || !w_k || !v_k || !den_j) return -1;
-    double* host = nullptr;
-    double* dev = cached_scratch((size_t)3 * n + m, &host);
-    if (!dev) return -2;
-    const auto A = lat_from(a);
-    const auto g = geom(l, m, n, nx, ny);
-    hipLaunchKernelGGL(varm_planes_k<real_t>, dim3(n), dim3(kRedThreads), 0, abi_stream(), A, g, cte1, dev);
-    report_launch("varm_planes_k");
-    hipLaunchKernelGGL(varm_planes_j<real_t>, dim3(m), dim3(kRedThreads), 0, abi_stream(), A, g, cte1,
-                       dev + 3 * n);
-    report_launch("varm_planes_j");
-    if (int rc = fetch(dev, host, (size_t)3 * n + m)) return rc;
+    double *dev = nullptr, *host = nullptr;
+    const long rows = (long)m * n;
+    if (!cached_scratch((size_t)rows * 4, (size_t)3 * n + m, &dev, &host)) return -2;
+    hipLaunchKernelGGL(varm_rows<real_t>, dim3(ceil_div(rows, 4)), dim3(kRedThreads), 0, abi_stream(), lat_from(a),
+                       geom(l, m, n, nx, ny), cte1, dev);
+    report_launch("varm_rows");
+    hipLaunchKernelGGL(varm_fold, dim3(n + m), dim3(kRedThreads), 0, abi_stream(), dev, m, n, host);
+    report_launch("varm_fold");
+    if (int rc = finish()) return rc;
     // rvol = 1.0/(float(l)) in default real (SRC/varm.F90:94)
     const double rvol = (double)(real_t)(1.0f / (float)l);
     for (int k = 0; k < n; ++k) {
@@ -480,18 +488,17 @@ int draglift_gpu(real_t** a, const int* obs, int l, int m, int n, int nx, int ny
         std::fprintf(stderr, "bgk3d_gpu: draglift box [%d:%d,%d:%d,%d:%d] leaves the mask\n", is, ie, js, je, ks, ke);
         return -1;
     }
-    double* host = nullptr;
-    double* dev = cached_scratch((size_t)(kRedBlocks + 1) * 3, &host);
-    if (!dev) return -2;
+    double *dev = nullptr, *host = nullptr;
+    if (!cached_scratch((size_t)kRedBlocks * 3, 3, &dev, &host)) return -2;
     const long cells = (long)(ie - is + 1) * (je - js + 1) * (ke - ks + 1);
     const int nb = (int)((cells + kRedThreads - 1) / kRedThreads < kRedBlocks ? (cells + kRedThreads - 1) / kRedThreads
                                                                                 : kRedBlocks);
     hipLaunchKernelGGL(draglift_partial<real_t>, dim3(nb), dim3(kRedThreads), 0, abi_stream(), lat_from(a),
-                       geom(l, m, n, nx, ny), obs, is, ie, js, je, ks, ke, dev + 3);
+                       geom(l, m, n, nx, ny), obs, is, ie, js, je, ks, ke, dev);
     report_launch("draglift_partial");
-    hipLaunchKernelGGL(fold_partials<3>, dim3(1), dim3(kRedThreads), 0, abi_stream(), dev + 3, nb, dev);
+    hipLaunchKernelGGL(fold_partials<3>, dim3(1), dim3(kRedThreads), 0, abi_stream(), dev, nb, host);
     report_launch("fold_partials");
-    if (int rc = fetch(dev, host, 3)) return rc;
+    if (int rc = finish()) return rc;
     // norm = uno/(u_inflow*u_inflow*radius) in the storage kind (:178)
     const real_t norm = real_t(1) / (u_inflow * u_inflow * (real_t)radius);
     for (int q = 0; q < 3; ++q) out[q] = host[q] * (double)norm;
@@ -508,16 +515,15 @@ static int line_profile(real_t** a, int l, int m, int n, int nx, int ny, int axi
     if (!shape_ok("line profile", l, m, n, nx, ny, a) || !out) return -1;
     if (count <= 0 || first < 1 || first + count - 1 > len) return -1;
     if (c1 < 0 || c1 > lim1 + 1 || c2 < 0 || c2 > lim2 + 1) return -1;
-    double* host = nullptr;
+    double *dev = nullptr, *host = nullptr;
     const size_t bytes = (size_t)4 * count * sizeof(real_t);
-    double* dev = cached_scratch((bytes + sizeof(double) - 1) / sizeof(double), &host);
-    if (!dev) return -2;
-    real_t* d = reinterpret_cast<real_t*>(dev);
+    if (!cached_scratch(0, (bytes + sizeof(double) - 1) / sizeof(double), &dev, &host)) return -2;
+    real_t* line = reinterpret_cast<real_t*>(host);
     hipLaunchKernelGGL(prof_line_kernel<real_t>, dim3(ceil_div(count, 64)), dim3(64), 0, abi_stream(), lat_from(a),
-                       geom(l, m, n, nx, ny), axis, c1, c2, first, count, cte1, d);
+                       geom(l, m, n, nx, ny), axis, c1, c2, first, count, cte1, line);
     report_launch("prof_line_kernel");
-    BGK_HIP_CHECK(hipMemcpyAsync(out, d, bytes, hipMemcpyDeviceToHost, abi_stream()));
-    BGK_HIP_CHECK(hipStreamSynchronize(abi_stream()));
+    if (int rc = finish()) return rc;
+    std::memcpy(out, line, bytes);
     return 0;
 }
 
