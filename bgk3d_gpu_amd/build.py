@@ -73,7 +73,7 @@ def build_one(name: str, sources, extra, verbose=False) -> Path:
         for j in jobs:
             j.result()
         lib = out.with_suffix(".so.tmp")
-        _hipcc([hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", str(lib)], name, verbose)
+        _hipcc([hipcc(), "-shared", "-fPIC", "-pthread", f"--offload-arch={ARCH}", *objs, "-o", str(lib)], name, verbose)
         os.replace(lib, out)
     return out
 

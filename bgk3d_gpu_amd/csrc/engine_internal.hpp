@@ -54,6 +54,9 @@ struct bgk_handle {
     int8_t* omask = nullptr;
     double* scratch = nullptr;
     double* hscratch = nullptr;
+    // device and pinned host staging of bgk_fields, from its first call on
+    void *stage = nullptr, *hstage = nullptr;
+    size_t stage_bytes = 0;
     long long steps = 0;
     bool borrowed = false;  // lattice memory, scratch and stream belong to a server
     std::vector<hipEvent_t> events;

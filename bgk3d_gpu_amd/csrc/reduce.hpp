@@ -262,28 +262,27 @@ __global__ void prof_line_kernel(Lattice19<S> a, Geometry g, int axis, int c1, i
     out[4 * t + 3] = den;
 }
 
-// Interior macroscopic fields (rho, ux, uy, uz) in FP64, i fastest; the
-// moments are formed in the collision kind with the reference's order.
+// Macroscopic fields of `count` interior cells from cell `first` on (i fastest):
+// rho, ux, uy, uz in the collision kind, with the reference's order, at out +
+// q * count for each field q whose bit is set in `want`, one after the other.
 template <typename S>
-__global__ void fields_kernel(Lattice19<S> a, Geometry g, typename Storage<S>::compute cte1,
-                              double* __restrict__ rho, double* __restrict__ ux, double* __restrict__ uy,
-                              double* __restrict__ uz)
+__global__ void fields_kernel(Lattice19<S> a, Geometry g, typename Storage<S>::compute cte1, long first, int count,
+                              int want, typename Storage<S>::compute* __restrict__ out)
 {
     typedef typename Storage<S>::compute R;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long cells = (long)g.l * g.m * g.n;
-    if (t >= cells) return;
+    const int u = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (u >= count) return;
+    const long t = first + u;
     const int i = 1 + (int)(t % g.l), j = 1 + (int)((t / g.l) % g.m), k = 1 + (int)(t / ((long)g.l * g.m));
-    const long s = gidx(g, i, j, k);
     R x[19];
-#pragma unroll
-    for (int d = 0; d < 19; ++d) x[d] = Storage<S>::load(a.p[d] + s);
+    load_cell(a, gidx(g, i, j, k), x);
     const R r = density_ref(x, cte1);
     const R rinv = R(1) / r;
-    if (rho) rho[t] = (double)r;
-    if (ux) ux[t] = (double)((x[0] + x[1] + x[2] + x[3] + x[4] - x[9] - x[10] - x[11] - x[12] - x[13]) * rinv);
-    if (uy) uy[t] = (double)((x[2] + x[6] + x[7] + x[8] + x[11] - x[0] - x[9] - x[15] - x[16] - x[17]) * rinv);
-    if (uz) uz[t] = (double)((x[3] + x[5] + x[6] + x[12] + x[17] - x[1] - x[8] - x[10] - x[14] - x[15]) * rinv);
+    R* to = out + u;
+    if (want & 1) *to = r, to += count;
+    if (want & 2) *to = (x[0] + x[1] + x[2] + x[3] + x[4] - x[9] - x[10] - x[11] - x[12] - x[13]) * rinv, to += count;
+    if (want & 4) *to = (x[2] + x[6] + x[7] + x[8] + x[11] - x[0] - x[9] - x[15] - x[16] - x[17]) * rinv, to += count;
+    if (want & 8) *to = (x[3] + x[5] + x[6] + x[12] + x[17] - x[1] - x[8] - x[10] - x[14] - x[15]) * rinv;
 }
 
 // Interior of one population array <-> FP64 buffer (i fastest).
