@@ -35,6 +35,10 @@ __device__ __forceinline__ long gidx(const Geometry& g, int i, int j, int k)
 // Boundary faces.  A(d) is population d (1-based, as in the Fortran).
 // -------------------------------------------------------------------------
 #define BGK_A(d, i, j, k) a.p[(d)-1][gidx(g, (i), (j), (k))]
+// Every face cell below reads all its values before it writes any: the
+// compiler has to keep a load behind an earlier store (they may alias), and
+// ten dependent round trips made driven_faces 13 us at 64^3, whatever its size.
+
 // bcond_driven x faces at (j, k), j=1..m, k=1..n (SRC/bcond.driven.F90:105-119).
 // The y and z faces are written in the same launch (driven_faces), so the
 // writes they overwrite (the same population of the same halo cell) are
@@ -46,16 +50,19 @@ __device__ __forceinline__ void driven_x_cell(Lattice19<R>& a, const Geometry& g
     const int l = g.l, l1 = g.l + 1;
     const bool y_lo = j == 1, y_hi = j == g.m;  // the y faces rewrite these
     const bool z_lo = k == 1, z_hi = k == g.n;  // the z faces rewrite these
-    if (!y_lo) BGK_A(12, l1, j - 1, k) = BGK_A(1, l, j, k);
-    if (!z_lo) BGK_A(13, l1, j, k - 1) = BGK_A(2, l, j, k);
-    if (!y_hi) BGK_A(10, l1, j + 1, k) = BGK_A(3, l, j, k);
-    if (!z_hi) BGK_A(11, l1, j, k + 1) = BGK_A(4, l, j, k);
-    BGK_A(14, l1, j, k) = BGK_A(5, l, j, k);
-    if (!y_lo) BGK_A(3, 0, j - 1, k) = BGK_A(10, 1, j, k);
-    if (!z_lo) BGK_A(4, 0, j, k - 1) = BGK_A(11, 1, j, k);
-    if (!y_hi) BGK_A(1, 0, j + 1, k) = BGK_A(12, 1, j, k);
-    if (!z_hi) BGK_A(2, 0, j, k + 1) = BGK_A(13, 1, j, k);
-    BGK_A(5, 0, j, k) = BGK_A(14, 1, j, k);
+    const R v1 = BGK_A(1, l, j, k), v2 = BGK_A(2, l, j, k), v3 = BGK_A(3, l, j, k), v4 = BGK_A(4, l, j, k),
+            v5 = BGK_A(5, l, j, k), v10 = BGK_A(10, 1, j, k), v11 = BGK_A(11, 1, j, k), v12 = BGK_A(12, 1, j, k),
+            v13 = BGK_A(13, 1, j, k), v14 = BGK_A(14, 1, j, k);
+    if (!y_lo) BGK_A(12, l1, j - 1, k) = v1;
+    if (!z_lo) BGK_A(13, l1, j, k - 1) = v2;
+    if (!y_hi) BGK_A(10, l1, j + 1, k) = v3;
+    if (!z_hi) BGK_A(11, l1, j, k + 1) = v4;
+    BGK_A(14, l1, j, k) = v5;
+    if (!y_lo) BGK_A(3, 0, j - 1, k) = v10;
+    if (!z_lo) BGK_A(4, 0, j, k - 1) = v11;
+    if (!y_hi) BGK_A(1, 0, j + 1, k) = v12;
+    if (!z_hi) BGK_A(2, 0, j, k + 1) = v13;
+    BGK_A(5, 0, j, k) = v14;
 }
 
 // bcond_driven y faces at (i, k), i=1..l, k=1..n (SRC/bcond.driven.F90:169-183);
@@ -66,16 +73,19 @@ __device__ __forceinline__ void driven_y_cell(Lattice19<R>& a, const Geometry& g
 {
     const int m = g.m, m1 = g.m + 1;
     const bool z_lo = k == 1, z_hi = k == g.n;
-    BGK_A(8, i, 0, k) = BGK_A(17, i, 1, k);
-    BGK_A(12, i + 1, 0, k) = BGK_A(1, i, 1, k);
-    BGK_A(3, i - 1, 0, k) = BGK_A(10, i, 1, k);
-    if (!z_lo) BGK_A(7, i, 0, k - 1) = BGK_A(16, i, 1, k);
-    if (!z_hi) BGK_A(9, i, 0, k + 1) = BGK_A(18, i, 1, k);
-    BGK_A(10, i + 1, m1, k) = BGK_A(3, i, m, k);
-    if (!z_hi) BGK_A(16, i, m1, k + 1) = BGK_A(7, i, m, k);
-    BGK_A(17, i, m1, k) = BGK_A(8, i, m, k);
-    if (!z_lo) BGK_A(18, i, m1, k - 1) = BGK_A(9, i, m, k);
-    BGK_A(1, i - 1, m1, k) = BGK_A(12, i, m, k);
+    const R v17 = BGK_A(17, i, 1, k), v1 = BGK_A(1, i, 1, k), v10 = BGK_A(10, i, 1, k), v16 = BGK_A(16, i, 1, k),
+            v18 = BGK_A(18, i, 1, k), v3 = BGK_A(3, i, m, k), v7 = BGK_A(7, i, m, k), v8 = BGK_A(8, i, m, k),
+            v9 = BGK_A(9, i, m, k), v12 = BGK_A(12, i, m, k);
+    BGK_A(8, i, 0, k) = v17;
+    BGK_A(12, i + 1, 0, k) = v1;
+    BGK_A(3, i - 1, 0, k) = v10;
+    if (!z_lo) BGK_A(7, i, 0, k - 1) = v16;
+    if (!z_hi) BGK_A(9, i, 0, k + 1) = v18;
+    BGK_A(10, i + 1, m1, k) = v3;
+    if (!z_hi) BGK_A(16, i, m1, k + 1) = v7;
+    BGK_A(17, i, m1, k) = v8;
+    if (!z_lo) BGK_A(18, i, m1, k - 1) = v9;
+    BGK_A(1, i - 1, m1, k) = v12;
 }
 
 // bcond_driven z faces + lid, i=1..l, j=1..m (SRC/bcond.driven.F90:233-247);
@@ -85,24 +95,19 @@ template <typename R>
 __device__ __forceinline__ void walls_z_cell(Lattice19<R>& a, const Geometry& g, int i, int j, R force, int lid)
 {
     const int n = g.n, n1 = g.n + 1;
-    BGK_A(6, i, j, 0) = BGK_A(15, i, j, 1);
-    BGK_A(4, i - 1, j, 0) = BGK_A(11, i, j, 1);
-    BGK_A(7, i, j - 1, 0) = BGK_A(16, i, j, 1);
-    BGK_A(13, i + 1, j, 0) = BGK_A(2, i, j, 1);
-    BGK_A(18, i, j + 1, 0) = BGK_A(9, i, j, 1);
-    BGK_A(15, i, j, n1) = BGK_A(6, i, j, n);
-    if (lid) {
-        BGK_A(2, i - 1, j, n1) = BGK_A(13, i, j, n) + force;
-    } else {
-        BGK_A(2, i - 1, j, n1) = BGK_A(13, i, j, n);
-    }
-    BGK_A(9, i, j - 1, n1) = BGK_A(18, i, j, n);
-    if (lid) {
-        BGK_A(11, i + 1, j, n1) = BGK_A(4, i, j, n) - force;
-    } else {
-        BGK_A(11, i + 1, j, n1) = BGK_A(4, i, j, n);
-    }
-    BGK_A(16, i, j + 1, n1) = BGK_A(7, i, j, n);
+    const R v15 = BGK_A(15, i, j, 1), v11 = BGK_A(11, i, j, 1), v16 = BGK_A(16, i, j, 1), v2 = BGK_A(2, i, j, 1),
+            v9 = BGK_A(9, i, j, 1), v6 = BGK_A(6, i, j, n), v13 = BGK_A(13, i, j, n), v18 = BGK_A(18, i, j, n),
+            v4 = BGK_A(4, i, j, n), v7 = BGK_A(7, i, j, n);
+    BGK_A(6, i, j, 0) = v15;
+    BGK_A(4, i - 1, j, 0) = v11;
+    BGK_A(7, i, j - 1, 0) = v16;
+    BGK_A(13, i + 1, j, 0) = v2;
+    BGK_A(18, i, j + 1, 0) = v9;
+    BGK_A(15, i, j, n1) = v6;
+    BGK_A(2, i - 1, j, n1) = lid ? v13 + force : v13;
+    BGK_A(9, i, j - 1, n1) = v18;
+    BGK_A(11, i + 1, j, n1) = lid ? v4 - force : v4;
+    BGK_A(16, i, j + 1, n1) = v7;
 }
 
 // bcond_driven in one launch: threads [0, m*n) take the x faces, the next
@@ -195,19 +200,21 @@ template <typename R, bool WALLS, bool XP = true>
 __device__ __forceinline__ void y_face_part(Lattice19<R>& a, const Geometry& g, int i, int k)
 {
     const int si = halo_side(i, g.l), sk = halo_side(k, g.n);
+    R v[10];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int jt = h == 0 ? 0 : g.m + 1, js = h == 0 ? g.m : 1;
+    for (int q = 0; q < 10; ++q) {
+        const int d = q < 5 ? kEnterYlo[q] : kEnterYhi[q - 5], js = q < 5 ? g.m : 1;
+        const int is = XP && enters(si, cx_of(d)) ? wrap_to(si, g.l) : i;
+        v[q] = a.p[d][gidx(g, is, js, k)];
+    }
 #pragma unroll
-        for (int q = 0; q < 5; ++q) {
-            const int d = h == 0 ? kEnterYlo[q] : kEnterYhi[q];
-            if (enters(sk, cz_of(d))) {
-                if (!WALLS) continue;                                 // the z face writes it later
-                if (i + cx_of(d) >= 1 && i + cx_of(d) <= g.l) continue;  // a wall writes it later
-            }
-            const int is = XP && enters(si, cx_of(d)) ? wrap_to(si, g.l) : i;
-            a.p[d][gidx(g, i, jt, k)] = a.p[d][gidx(g, is, js, k)];
+    for (int q = 0; q < 10; ++q) {
+        const int d = q < 5 ? kEnterYlo[q] : kEnterYhi[q - 5], jt = q < 5 ? 0 : g.m + 1;
+        if (enters(sk, cz_of(d))) {
+            if (!WALLS) continue;                                 // the z face writes it later
+            if (i + cx_of(d) >= 1 && i + cx_of(d) <= g.l) continue;  // a wall writes it later
         }
+        a.p[d][gidx(g, i, jt, k)] = v[q];
     }
 }
 
@@ -217,16 +224,18 @@ template <typename R, bool XP = true>
 __device__ __forceinline__ void z_face_part(Lattice19<R>& a, const Geometry& g, int i, int j)
 {
     const int si = halo_side(i, g.l), sj = halo_side(j, g.m);
+    R v[10];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int kt = h == 0 ? 0 : g.n + 1, ks = h == 0 ? g.n : 1;
+    for (int q = 0; q < 10; ++q) {
+        const int d = q < 5 ? kEnterZlo[q] : kEnterZhi[q - 5], ks = q < 5 ? g.n : 1;
+        const int is = XP && enters(si, cx_of(d)) ? wrap_to(si, g.l) : i;
+        const int js = enters(sj, cy_of(d)) ? wrap_to(sj, g.m) : j;
+        v[q] = a.p[d][gidx(g, is, js, ks)];
+    }
 #pragma unroll
-        for (int q = 0; q < 5; ++q) {
-            const int d = h == 0 ? kEnterZlo[q] : kEnterZhi[q];
-            const int is = XP && enters(si, cx_of(d)) ? wrap_to(si, g.l) : i;
-            const int js = enters(sj, cy_of(d)) ? wrap_to(sj, g.m) : j;
-            a.p[d][gidx(g, i, j, kt)] = a.p[d][gidx(g, is, js, ks)];
-        }
+    for (int q = 0; q < 10; ++q) {
+        const int d = q < 5 ? kEnterZlo[q] : kEnterZhi[q - 5];
+        a.p[d][gidx(g, i, j, q < 5 ? 0 : g.n + 1)] = v[q];
     }
 }
 
@@ -374,15 +383,20 @@ __global__ void obstacle_bb(Lattice19<R> a, Geometry g, const int* __restrict__ 
     };
     if (!visited_solid(i, j, k)) return;
     const long c = gidx(g, i, j, k);
+    R v[18];
+    uint32_t write = 0;
 #pragma unroll
     for (int d = 0; d < 18; ++d) {
         // reference: a_d(i,j,k) = a_opp(d)(i + c_d)
         const int dx = cx_of(d), dy = cy_of(d), dz = cz_of(d);
         // the neighbour precedes (i,j,k) in the loop order (k, then j, then i)
         const bool earlier = dz < 0 || (dz == 0 && (dy < 0 || (dy == 0 && dx < 0)));
-        if (earlier && visited_solid(i + dx, j + dy, k + dz)) continue;
-        a.p[d][c] = a.p[opp_of(d)][gidx(g, i + dx, j + dy, k + dz)];
+        v[d] = a.p[opp_of(d)][gidx(g, i + dx, j + dy, k + dz)];
+        if (!(earlier && visited_solid(i + dx, j + dy, k + dz))) write |= 1u << d;
     }
+#pragma unroll
+    for (int d = 0; d < 18; ++d)
+        if ((write >> d) & 1u) a.p[d][c] = v[d];
 }
 
 #undef BGK_A
