@@ -28,7 +28,13 @@
 // plane) it takes 235.  Loads issued two planes ahead, or before the first
 // step instead of after it, gave no more; plain stores 290, 6 waves and two
 // blocks per CU 305, tiles in launch order over the XCDs 361.  FP64 at 192^3:
-// 227 (359).
+// 207 (359).
+//
+// Where at most 32 cells of a row are left, tiles of 32 cells with two rows
+// per wave take them (half the waves of a 64-cell tile that is mostly empty):
+// LES FP32 201 x 135 x 99 61 -> 56 us per step, FP32 87^3 18.4 -> 15.9, 130^3
+// 50.0 -> 48.3, FP64 75^3 27.0 -> 22.8; 16 cells would no longer write whole
+// FP32 lines.
 //
 // Each step is the one-step kernels' arithmetic on the same values, rounded
 // to the storage type in between, so two steps here give the same bits as
@@ -47,11 +53,12 @@ namespace bgk {
 
 constexpr int kTileX = 64;
 
-// The tiles of a launch: tx * ty columns of th rows, each cut into cz ranges
-// of zc planes.
+// The tiles of a launch: tx * ty columns of 64 cells x th rows and, where the
+// last 1 ... 32 cells of a row are left, ty2 columns of 32 cells x 2 th rows;
+// each cut into cz ranges of zc planes.
 struct PairGrid {
-    int tx, ty, th, cz, zc;
-    int total;  // tx * ty * cz
+    int tx, ty, th, ty2, cz, zc;
+    int total;  // (tx * ty + ty2) * cz
 };
 
 // Barrier of the block for LDS only: global loads stay in flight across it
@@ -236,54 +243,65 @@ struct PairShape {
     static constexpr bool wide = std::is_same<typename Storage<S>::compute, double>::value;
     static constexpr int TY = sizeof(S) == 8 ? 8 : (wide ? 9 : 13);
     static constexpr bool DB = sizeof(S) < 8;
+    static constexpr int POP = (TY + 2) * (kTileX + 2);  // LDS elements per population
 };
 
 // The forms that take two steps per launch where that is faster (prefer_pair).
 template <typename S, int FMODE>
 constexpr bool kPairs = sizeof(S) >= 4 && !(PairShape<S>::wide && (FMODE & 4) != 0);
 
-// Two steps of one tile.  `seed`, `seed2`: the two steps' rounding seeds.
-template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, int SR>
-__device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid& g, int tile, uint32_t seed,
-                                          uint32_t seed2)
+// Two steps of the tile of 64 / RW cells x th rows whose first cell is (x0, j0,
+// k0); with RW = 2 a wave holds two rows.  `lone`: the tile spans the row.
+// `seed`, `seed2`: the two steps' rounding seeds.
+template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, int SR, int RW>
+__device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typename BitsOf<sizeof(S)>::type* lds, int x0,
+                                          int j0, int k0, int th, int zc, bool lone, uint32_t seed, uint32_t seed2)
 {
     constexpr int TY = PairShape<S>::TY;
     constexpr bool DB = PairShape<S>::DB;
     typedef typename Storage<S>::compute C;
     constexpr long ES = (long)sizeof(S);
-    constexpr int ROWS = TY + 2, PITCH = kTileX + 2, POP = ROWS * PITCH, BUF = 16 * POP;
+    constexpr int TILE = kTileX / RW, ROWS = TY + 2, PITCH = TILE + 2, POP = PairShape<S>::POP, BUF = 16 * POP;
+    static_assert((RW * TY + 2) * PITCH <= POP && 2 * (RW * TY + 2) <= 64, "LDS rows and side lanes");
     constexpr bool ZWALL = BZ == AX_WALL || BZ == AX_LID;
     constexpr bool BOUNCE = BX == AX_WALL || BY == AX_WALL || OBST;  // bounces that differ between lanes
     typedef typename BitsOf<sizeof(S)>::type Bits;
-    __shared__ Bits lds_[(DB ? 2 : 1) * BUF];
-    BGK_LDS Bits* const lds = (BGK_LDS Bits*)lds_;
 
-    const int x0 = 1 + (tile % g.tx) * kTileX;
-    const int j0 = 1 + (tile / g.tx % g.ty) * g.th;
-    const int k0 = 1 + (tile / (g.tx * g.ty)) * g.zc;
-    const int k1 = k0 + g.zc - 1 < p.n ? k0 + g.zc - 1 : p.n;
+    const int k1 = k0 + zc - 1 < p.n ? k0 + zc - 1 : p.n;
     const int first = ZWALL && k0 == 1 ? 1 : k0 - 1, last = k1 + 1;
     const int end1 = ZWALL && last > p.n ? p.n : last;  // last plane of the first step
 
-    // The thread's cell of the first step: LDS row r (0 and TY + 1 around
+    // The thread's cell of the first step: LDS row r (0 and rows + 1 around
     // the tile), column c (0 and width + 1 around it).  Lanes past the row's
-    // end or past the side columns repeat another lane's cell, so no lane is
-    // masked; cells outside a wall are computed on a cell inside and unused.
+    // end, past the last row or past the side columns repeat another lane's
+    // cell, so no lane is masked; cells outside a wall are computed on a cell
+    // inside and unused.  With two rows per wave, wave 0 holds the rows below
+    // and above the tile.
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
-    const int width = p.l - x0 + 1 < kTileX ? p.l - x0 + 1 : kTileX;
+    const int width = p.l - x0 + 1 < TILE ? p.l - x0 + 1 : TILE;
+    const int rows = p.m - j0 + 1 < th ? p.m - j0 + 1 : th;
+    const int col = lane & (TILE - 1);
     const bool side = wave == ROWS;
-    const int r = side ? (lane < 2 * (g.th + 2) ? lane >> 1 : 0) : wave;
-    const int c = side ? ((lane & 1) ? width + 1 : 0) : (lane < width ? lane + 1 : width);
-    const int jr = j0 - 1 + wave;  // the row of a wave that is not `side`
-    const bool out = !side && wave >= 1 && wave <= g.th && jr <= p.m;
-    const bool helps = side ? !(BX == AX_WALL && g.tx == 1)
-                            : wave <= g.th + 1 && (BY == AX_WALL ? jr >= 1 && jr <= p.m : jr <= p.m + 1);
+    const int jr = j0 - 1 + wave;  // RW = 1: the row of a wave that is not `side`
+    int r = wave;
+    bool out = !side && wave >= 1 && wave <= rows;
+    bool helps = side ? !(BX == AX_WALL && lone)
+                      : wave <= rows + 1 && (BY == AX_WALL ? jr >= 1 && jr <= p.m : jr <= p.m + 1);
+    if constexpr (RW == 2) {
+        r = wave == 0 ? (lane < TILE ? 0 : rows + 1) : 2 * wave - 1 + (lane < TILE ? 0 : 1);
+        if (wave != 0 && r > rows) r -= 1;
+        out = !side && wave >= 1 && 2 * wave - 1 <= rows;
+        helps = side ? helps : wave == 0;
+    }
+    if (side) r = lane < 2 * (rows + 2) ? lane >> 1 : 0;
+    const int c = side ? ((lane & 1) ? width + 1 : 0) : (col < width ? col + 1 : width);
     int i = x0 - 1 + c, j = j0 - 1 + r, face = 0;
     if (i < 1 || i > p.l) {
         if (BX == AX_HALO) face = i < 1 ? 1 : 2;
         i = (BX == AX_PERIODIC) == (i < 1) ? p.l : 1;
     }
     if (j < 1 || j > p.m) j = j < 1 ? p.m : (j == p.m + 1 ? 1 : p.m);
+    const int jout = RW == 2 ? j : jr;  // the row of an `out` wave's lane, scalar with one row per wave
     const int at = r * PITCH + c;
 
     // Pulls of the first step: population d of plane k at base(d) + a 32-bit
@@ -304,8 +322,8 @@ __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid&
     };
     // Obstacle links of the cell in plane k; only rows and planes of the box
     // look (the same for a whole wave).
-    const bool boxed = OBST && x0 + kTileX >= p.oi0 && x0 - 1 < p.oi0 + p.oni && j0 - 1 < p.oj0 + p.onj &&
-                       j0 + g.th >= p.oj0;
+    const bool boxed = OBST && x0 + TILE >= p.oi0 && x0 - 1 < p.oi0 + p.oni && j0 - 1 < p.oj0 + p.onj &&
+                       j0 + th >= p.oj0;
     auto links = [&](int k) -> uint32_t {
         const unsigned ri = (unsigned)(i - p.oi0), rj = (unsigned)(j - p.oj0), rk = (unsigned)(k - p.ok0);
         if (ri < (unsigned)p.oni && rj < (unsigned)p.onj && rk < (unsigned)p.onk)
@@ -422,7 +440,7 @@ __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid&
     uint32_t ob1 = 0;  // link mask in plane kk - 1
     constexpr int UP[5] = {3, 5, 6, 12, 17}, DN[5] = {10, 14, 15, 1, 8};
     const int lend = p.lend > p.l ? p.lend : p.l;
-    const int ic = x0 + lane < lend ? x0 + lane : lend;
+    const int ic = x0 + col < lend ? x0 + col : lend;
     const uint32_t live = ic <= p.l ? ~0u : 0u;
     const uint32_t to = (uint32_t)(((long)j * p.nx + ic) * ES);
 
@@ -433,13 +451,13 @@ __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid&
         BGK_LDS Bits* buf = buffer(kk);
         S v[19];
         const uint32_t ob0 = ob;
-        const int iw = (int)lane_offset((uint32_t)i);
+        const int iw = (int)lane_offset((uint32_t)i), jo = RW == 2 ? (int)lane_offset((uint32_t)jout) : jout;
         if constexpr (S1) {
             step_one(kk, buf, v);
             if constexpr (BOUNCE || ZWALL) {  // bounced pulls of plane kk from below: own populations going down
                 for (int q = 0; q < 5; ++q) {
                     const int d = UP[q];
-                    if ((ZWALL && kk == 1) || wall(d, iw, jr) || (OBST && ((ob0 >> d) & 1u))) up[q] = v[DN[q]];
+                    if ((ZWALL && kk == 1) || wall(d, iw, jo) || (OBST && ((ob0 >> d) & 1u))) up[q] = v[DN[q]];
                 }
             }
             if (kk < end1) fetch(kk + 1);
@@ -468,7 +486,7 @@ __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid&
                         else
                             w = get(dc);
                         if constexpr (BOUNCE)
-                            if (wall(d, iw, jr) || (OBST && ((ob1 >> d) & 1u))) w = ups[q];
+                            if (wall(d, iw, jo) || (OBST && ((ob1 >> d) & 1u))) w = ups[q];
                     }
                 }
                 x[d] = Storage<S>::widen(w);
@@ -493,7 +511,7 @@ __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid&
                     if constexpr (d != 18) {
                         w = get(dc);
                         if constexpr (BOUNCE)
-                            if (wall(d, iw, jr) || (OBST && ((ob0 >> d) & 1u))) w = v[opp_of(d)];
+                            if (wall(d, iw, jo) || (OBST && ((ob0 >> d) & 1u))) w = v[opp_of(d)];
                     }
                     mid[place(kMid, d)] = w;
                 } else if constexpr (cz_of(d) > 0) {
@@ -524,6 +542,25 @@ __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid&
     if (end1 < last) advance(last, F{}, T{});
 }
 
+// Two steps of one tile of the launch.
+template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, int SR>
+__device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid& g, int tile, uint32_t seed,
+                                          uint32_t seed2)
+{
+    typedef typename BitsOf<sizeof(S)>::type Bits;
+    __shared__ Bits lds_[(PairShape<S>::DB ? 2 : 1) * 16 * PairShape<S>::POP];
+    BGK_LDS Bits* const lds = (BGK_LDS Bits*)lds_;
+    const int per = g.tx * g.ty + g.ty2, q = tile % per;
+    const int k0 = 1 + (tile / per) * g.zc;
+    const bool lone = g.tx + (g.ty2 ? 1 : 0) == 1;
+    if (q < g.tx * g.ty)
+        pair_rows<S, BX, BY, BZ, OBST, FMODE, SR, 1>(p, lds, 1 + q % g.tx * kTileX, 1 + q / g.tx * g.th, k0, g.th, g.zc,
+                                                     lone, seed, seed2);
+    else
+        pair_rows<S, BX, BY, BZ, OBST, FMODE, SR, 2>(p, lds, 1 + g.tx * kTileX, 1 + (q - g.tx * g.ty) * 2 * g.th, k0,
+                                                     2 * g.th, g.zc, lone, seed, seed2);
+}
+
 // Block x of n blocks as the b-th tile: consecutive tiles on one XCD (blocks
 // go to the 8 XCDs in turn).  May return n or more: no tile.
 __device__ __forceinline__ int xcd_tile(int x, int n)
@@ -541,28 +578,37 @@ __global__ __launch_bounds__(64 * (PairShape<S>::TY + 3)) void collide_pair(Fuse
 
 // Tiles of an l x m x n lattice with at most `rows` rows: the rows and planes
 // per block that minimise `cost`, the time of a launch in units of one row of
-// 64 cells taken one plane on.  A block takes zc + 2 planes of th + 2 rows;
-// the fit of 394 FP32 launches (64^3 ... 256^3, th 3 ... 13) has smaller
-// constants, since the border rows and first planes do less.  `cus`
-// blocks run at a time (256, one per CU, in a launch of its own); a last round that is partly empty costs about half of a full
-// one, the full ones being bound by HBM.  The choice made was within 4 % of
-// the fastest on average over 8 sizes, at most 9 %.
+// 64 cells taken one plane on.  A block takes zc + 2 planes of th + 2 rows
+// (a fit has smaller constants, since the border rows and first planes do
+// less); `cus` blocks run at a time (256, one per CU, in a launch of its own).
+// One round of blocks is worth a lot: tiles that walk up together share their
+// border reads in L2 and no CU waits for a block to start, so two full rounds
+// cost 2.3 of one, and a launch of 257 blocks 1.7 (900 x 150^2 FP32, per
+// step: 247 blocks 323 us, the same columns cut in two 365, in five 376;
+// 400^3: 241 blocks 1030 us, 404 1359, 1010 1230).  The weights fit 45 such
+// launches (256^3, 400^3, 512^3, 900 x 150^2) to 8 %.
 inline PairGrid pair_grid(int l, int m, int n, int rows, double& cost, double cus = 256)
 {
     PairGrid g{};
-    g.tx = ceil_div(l, kTileX);
+    const int left = l % kTileX;
+    const bool tail = left > 0 && left <= kTileX / 2;
+    g.tx = l / kTileX + (left > kTileX / 2 ? 1 : 0);
     cost = -1;
     for (int th = std::min(m, rows); th >= 1; --th) {
         const int ty = ceil_div(m, th);
         if (ceil_div(m, ty) != th) continue;  // as many tiles of fewer rows
         for (int zc = n, cz = 1;; cz = ceil_div(n, zc - 1), zc = ceil_div(n, cz)) {  // every distinct cut of n
-            const double blocks = (double)g.tx * ty * cz;
+            const int ty2 = tail ? ceil_div(m, 2 * th) : 0;
+            const double blocks = ((double)g.tx * ty + ty2) * cz;
             if (blocks >= 1u << 30) break;
-            const double c = 0.5 * (std::ceil(blocks / cus) + blocks / cus) * (zc + 1) * (th + 2.5);
+            const double rounds = blocks / cus;
+            const double c = (rounds <= 1 ? 0.9 + 0.1 * rounds : 0.55 * std::ceil(rounds) + 0.62 * rounds) * (zc + 1) *
+                             (th + 2.5);
             if (cost < 0 || c < cost) {
                 cost = c;
                 g.ty = ty;
                 g.th = th;
+                g.ty2 = ty2;
                 g.cz = cz;
                 g.zc = zc;
                 g.total = (int)blocks;

@@ -66,3 +66,24 @@ def test_pairs_match_single_steps(gpu, kw, storage, mixed):
             out.append(eng.populations())
     assert np.isfinite(out[0]).all() and np.any(out[0] != 0)
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("storage,mixed", [("f32", 0), ("f64", 0), ("f32", 2)])
+@pytest.mark.parametrize("name", ["ldc", "periodic", "channel", "inflow"])
+@pytest.mark.parametrize("size", [(32, 27, 3), (31, 1, 2), (33, 3, 4), (96, 53, 3), (95, 17, 5), (160, 19, 2)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_narrow_tiles_match_single_steps(gpu, size, name, storage, mixed):
+    """The tiles of 32 cells and two rows per wave that take a row's last 1 ... 32
+    cells: none but them, beside one or two of 64, one cell too many for them;
+    rows that end in the first or the second half of a wave, in a tile of
+    their own, or in a full tile."""
+    case = Case(l=size[0], m=size[1], n=size[2], **CASES[name])
+    print(f"[gpu] narrow tiles {name} {storage} mixed={mixed} {size}", flush=True)
+    out = []
+    for chunks in ((6,), (1,) * 6):
+        with Engine(case, storage, layout=1, mixed=mixed) as eng:
+            for c in chunks:
+                eng.step(c)
+            out.append(eng.populations())
+    assert np.isfinite(out[0]).all() and np.any(out[0] != 0)
+    assert np.array_equal(out[0], out[1])
