@@ -153,7 +153,7 @@ inline bool compute_double(const bgk_config& c) { return c.storage == BGK_F64 ||
 // launches: a single step takes 1.5 + its bytes at 6.2 TB/s, at least 4.6; a
 // pair 2.5 + its cost (pair_grid) times 0.42 in FP32 (0.37 ... 0.43 over
 // cavities, Taylor-Green, channel and the sphere, 64^3 ... 512^3), 0.46
-// in MIXED2 and 0.80 in FP64 (0.67 without walls).  Measured per step, one step a launch against
+// in MIXED2 and 0.70 in FP64 (0.63 ... 0.72).  Measured per step, one step a launch against
 // two: FP32 256^3 410 / 268, 192^3 175 / 112, 64^3 9.7 / 6.3, FP64 192^3 359 /
 // 227.  LES with FP64 arithmetic stays with one (152 against 143 at 201 x 135
 // x 99: more values live than registers), 16-bit storage too (118 against 108
@@ -170,7 +170,7 @@ inline bool prefer_pair(const bgk_config& c, long plane, PairGrid& g)
     g = pair_grid(c.l, c.m, c.n, rows, cost);
     const double cells = (double)c.l * c.m * c.n;
     const double two = 2 * std::max(4.6, 1.5 + 38.0 * (double)es * cells / 6.2e6);
-    return 2.5 + cost * (es == 8 ? 0.80 : (wide ? 0.46 : 0.42)) < two;
+    return 2.5 + cost * (es == 8 ? 0.70 : (wide ? 0.46 : 0.42)) < two;
 }
 
 // Validate `c` and fill the layout and the derived parameters of `h`

@@ -509,9 +509,12 @@ __device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typenam
                 if constexpr (cz_of(d) == 0) {
                     S w = v[18];
                     if constexpr (d != 18) {
-                        w = get(dc);
+                        // bounced: the own opposite value, from LDS too (kept in registers
+                        // across the barrier it cost spills: FP64 cavity 256^3 543 -> 469 us)
+                        int q = lds_slot(d) * POP + at - cy_of(d) * PITCH - cx_of(d);
                         if constexpr (BOUNCE)
-                            if (wall(d, iw, jo) || (OBST && ((ob0 >> d) & 1u))) w = v[opp_of(d)];
+                            if (wall(d, iw, jo) || (OBST && ((ob0 >> d) & 1u))) q = lds_slot(opp_of(d)) * POP + at;
+                        w = __builtin_bit_cast(S, (Bits)buf[q]);
                     }
                     mid[place(kMid, d)] = w;
                 } else if constexpr (cz_of(d) > 0) {
