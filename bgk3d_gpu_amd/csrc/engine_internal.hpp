@@ -153,16 +153,17 @@ inline bool compute_double(const bgk_config& c) { return c.storage == BGK_F64 ||
 // launches: a single step takes 1.5 + its bytes at 6.2 TB/s, at least 4.6; a
 // pair 2.5 + its cost (pair_grid) times 0.42 in FP32 (0.37 ... 0.43 over
 // cavities, Taylor-Green, channel and the sphere, 64^3 ... 512^3), 0.46
-// in MIXED2 and 0.70 in FP64 (0.63 ... 0.72).  Measured per step, one step a launch against
-// two: FP32 256^3 410 / 268, 192^3 175 / 112, 64^3 9.7 / 6.3, FP64 192^3 359 /
-// 227.  LES with FP64 arithmetic stays with one (152 against 143 at 201 x 135
-// x 99: more values live than registers), 16-bit storage too (118 against 108
-// for the FP16 channel at 512 x 128^2: bound by issue, half the bytes).
+// in MIXED2 and 0.70 in FP64 (0.63 ... 0.72); with LES 0.44, 0.53 and 1.10
+// (more values live than registers).  Measured per step, one step a launch
+// against two: FP32 256^3 410 / 268, 192^3 175 / 112, 64^3 9.7 / 6.3, FP64 192^3
+// 359 / 207; LES 128^3 MIXED2 60.7 / 47.5, FP64 109 / 95.  16-bit storage stays
+// with one: its kernels are bound by issue as much as by HBM (FP16 channel at
+// 512 x 128^2 108 / 118 with one cell per lane, 109 / 131 with two).
 inline bool prefer_pair(const bgk_config& c, long plane, PairGrid& g)
 {
     const size_t es = storage_bytes(c.storage);
     const bool wide = compute_double(c);
-    if (es < 4 || c.layout == 2 || (c.les && wide)) return false;
+    if (es < 4 || c.layout == 2) return false;
     // a lane's 32-bit byte offset spans up to four z levels (pair_tile)
     if (80.0 * (double)es * (double)plane >= 4.0e9) return false;
     double cost;
@@ -170,7 +171,8 @@ inline bool prefer_pair(const bgk_config& c, long plane, PairGrid& g)
     g = pair_grid(c.l, c.m, c.n, rows, cost);
     const double cells = (double)c.l * c.m * c.n;
     const double two = 2 * std::max(4.6, 1.5 + 38.0 * (double)es * cells / 6.2e6);
-    return 2.5 + cost * (es == 8 ? 0.70 : (wide ? 0.46 : 0.42)) < two;
+    const double us = es == 8 ? (c.les ? 1.10 : 0.70) : (wide ? (c.les ? 0.53 : 0.46) : (c.les ? 0.44 : 0.42));
+    return 2.5 + cost * us < two;
 }
 
 // Validate `c` and fill the layout and the derived parameters of `h`

@@ -14,7 +14,7 @@ template <typename S, int BX, int BY, int BZ, bool OB, int FM, int SR>
 void launch_fused(bgk_handle& h, bool pair)
 {
     const FusedArgs<S> p = fused_args<S>(h, h.cur, h.rest);
-    if constexpr (kPairs<S, FM>) {
+    if constexpr (kPairs<S>) {
         if (pair) {
             launch_pair<S, BX, BY, BZ, OB, FM, SR>(p, h.pgrid, h.stream);
             return;

@@ -246,9 +246,9 @@ struct PairShape {
     static constexpr int POP = (TY + 2) * (kTileX + 2);  // LDS elements per population
 };
 
-// The forms that take two steps per launch where that is faster (prefer_pair).
-template <typename S, int FMODE>
-constexpr bool kPairs = sizeof(S) >= 4 && !(PairShape<S>::wide && (FMODE & 4) != 0);
+// Storage types that take two steps per launch where that is faster (prefer_pair).
+template <typename S>
+constexpr bool kPairs = sizeof(S) >= 4;
 
 // Two steps of the tile of 64 / RW cells x th rows whose first cell is (x0, j0,
 // k0); with RW = 2 a wave holds two rows.  `lone`: the tile spans the row.

@@ -375,7 +375,7 @@ void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, int launch, 
         const BatchSlot<S>& sl = static_cast<const BatchSlot<S>*>(g.h_slots)[sb.single];
         FusedArgs<S> p = sl.args[launch & 1];
         p.seed = step_seed(sl.cfg_seed, sl.steps0 + t);
-        if constexpr (kPairs<S, 0>) {
+        if constexpr (kPairs<S>) {
             if (pair) {
                 launch_pair<S, AX_WALL, AX_WALL, AX_LID, false, 0, SR>(p, sl.pg, stream);
                 return;
@@ -399,7 +399,7 @@ void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, int launch, 
                            fused_block(rm), 0, stream, p, rm);
         return;
     }
-    if constexpr (kPairs<S, 0>) {
+    if constexpr (kPairs<S>) {
         if (pair) {
             hipLaunchKernelGGL((collide_pair_batched<S>), dim3((unsigned)pair_blocks((int)sb.ntiles)),
                                dim3(64 * (PairShape<S>::TY + 3)), 0, stream, d_slots, g.d_owner, sb.tile0,

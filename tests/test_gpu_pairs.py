@@ -87,3 +87,20 @@ def test_narrow_tiles_match_single_steps(gpu, size, name, storage, mixed):
             out.append(eng.populations())
     assert np.isfinite(out[0]).all() and np.any(out[0] != 0)
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("storage,mixed", [("f64", 0), ("f32", 2)])
+@pytest.mark.parametrize("kw", [dict(boundary="ldc"), dict(boundary="periodic", init=1),
+                                dict(boundary="inflow", obstacle=True)], ids=["ldc", "periodic", "inflow-obstacle"])
+def test_les_in_fp64_matches_single_steps(gpu, kw, storage, mixed):
+    """LES with FP64 arithmetic, in full and in narrow tiles."""
+    case = Case(l=70, m=30, n=24, svisc=0.01, u0=0.1, les=True, **kw)
+    print(f"[gpu] LES pairs {kw} {storage} mixed={mixed}", flush=True)
+    out = []
+    for chunks in ((8,), (1,) * 8):
+        with Engine(case, storage, layout=1, mixed=mixed) as eng:
+            for c in chunks:
+                eng.step(c)
+            out.append(eng.populations())
+    assert np.isfinite(out[0]).all() and np.any(out[0] != 0)
+    assert np.array_equal(out[0], out[1])
