@@ -9,9 +9,10 @@ collide, the reference's loop body (SRC/bgk3d.F90:169-196).
 
 value  = whole-job MLUPS = l*m*n*steps / time / 1e6 (SRC/finalize.F90:106-107)
 roofline: dominant kernel (the fused collide), algorithmic bytes per launch =
-          38 * 4 B * l*m*n (19 loads + 19 stores per interior cell), divided
-          by the kernel's average duration measured with hipEvents around each
-          launch in the timed region, against the 8 TB/s HBM peak.
+          38 * 4 B * l*m*n (19 loads + 19 stores per interior cell, once for
+          the two steps of a collide_pair launch), divided by the kernel's
+          average duration measured with hipEvents around each launch in the
+          timed region, against the 8 TB/s HBM peak.
 cpu_baseline: the reference's own Fortran CPU routines (oracle/_ref): its
           OpenMP loops on the host's cores, and its serial build, on a
           bounded sample of the same workload.
@@ -175,6 +176,12 @@ def bench_engine(case, storage, steps, warmup, want_ke=False, rounding=None, **k
     return total_ms, kern_ms, diag, info
 
 
+def steps_per_launch(case, info):
+    """2 where the engine takes two steps per launch (collide_pair): FP32 and
+    FP64 storage on padded rows (it chooses compact rows for one step)."""
+    return 2 if info["esize"] >= 4 and info["nx"] != case.l + 2 else 1
+
+
 def bench_sphere(steps):
     """Flow past a sphere, 1024 x 384 x 384 FP32 (Re = 300, R = 32 at
     (256, 192, 192), inflow 0.05, solid mask): the handle API, and the
@@ -187,9 +194,11 @@ def bench_sphere(steps):
     case = Case("inflow", l, m, n, svisc=U * 2 * R / 300.0, u0=U, obstacle=True)
     t, k, d, info = bench_engine(case, "f32", steps, 3, obstacle=2, centre=(l // 4, m // 2, n // 2), radius=R,
                                  u_inflow=U)
+    per = steps_per_launch(case, info)
     out = {"sphere_engine": {"mlups": round(case.cells * steps / (t * 1e-3) / 1e6, 1),
                              "collide_us": round(k * 1e3, 1), "device_bytes": info["bytes"],
-                             "alg_GBs": round(38 * 4 * case.cells / (k * 1e-3) / 1e9, 1),
+                             "steps_per_launch": per,
+                             "alg_GBs": round(38 * 4 * case.cells / (per * k * 1e-3) / 1e9, 1),
                              "workload": "sphere 1024x384x384 FP32, solid R=32, Re=300"}}
     log(f"sphere engine: {out['sphere_engine']}")
     ref_case = Case("inflow", l, m, n, svisc=0.02, u0=0.1, obstacle=True)
@@ -203,9 +212,8 @@ def bench_sphere(steps):
 
 def serving_ceiling(reqs, steps=200):
     """Upper bound on the mix's cell updates per second: every request at the
-    rate of one large (192^3) cavity of its storage type alone on the GPU,
-    which already streams at the HBM roofline -- the cell-weighted harmonic
-    mean of those rates.  No scheduler of these kernels can beat it."""
+    rate of one large (192^3) cavity of its storage type alone on the GPU --
+    the cell-weighted harmonic mean of those rates.  No scheduler of these kernels can beat it."""
     from bgk3d_gpu_amd import serving as S
     from bgk3d_gpu_amd.engine import Engine
 
@@ -257,7 +265,7 @@ def bench_serving(count, steps, budget_gb=32.0, load=0.8, min_cells=4 << 20, chu
         "throughput_ratio_vs_plain": r3(bat["throughput_mlups"] / plain["throughput_mlups"]),
         "throughput_ratio_vs_engine_loop": r3(bat["throughput_mlups"] / seq["throughput_mlups"]),
         "ceiling_mlups": round(ceiling, 1),
-        "ceiling_note": "every request at the rate of a 192^3 cavity of its storage alone (roofline-bound): "
+        "ceiling_note": "every request at the rate of a 192^3 cavity of its storage alone: "
                         + ", ".join(f"{k} {v:.0f}" for k, v in rates.items())
                         + " MLUPS; the 3x-the-plain-loop target would need "
                         + f"{3 * plain['throughput_mlups']:.0f}",
@@ -318,8 +326,9 @@ def main():
     ms_per_step = total_ms / args.steps
     mlups = case.cells * args.steps / (total_ms * 1e-3) / 1e6
     alg_bytes = 38 * s_bytes * case.cells
-    achieved = alg_bytes / (kern_avg_ms * 1e-3) / 1e9
-    log(f"MLUPS {mlups:.0f}; collide avg {kern_avg_ms * 1e3:.1f} us -> {achieved:.0f} GB/s")
+    per_launch = steps_per_launch(case, info)
+    achieved = alg_bytes / (per_launch * kern_avg_ms * 1e-3) / 1e9
+    log(f"MLUPS {mlups:.0f}; collide avg {kern_avg_ms * 1e3:.1f} us per step, {per_launch} per launch -> {achieved:.0f} GB/s")
     forms = {}
     if not args.no_forms:
         fsteps = max(10, args.steps // 4)
@@ -333,10 +342,11 @@ def main():
                                          ("f32_mixed2", "f32", 0, 4, 2)):
             if st == storage and not mixed:
                 continue
-            t, k, d, _ = bench_engine(case, st, fsteps, 5, rounding=rnd, mixed=mixed)
+            t, k, d, finfo = bench_engine(case, st, fsteps, 5, rounding=rnd, mixed=mixed)
+            per = steps_per_launch(case, finfo)
             forms[name] = {"mlups": round(case.cells * fsteps / (t * 1e-3) / 1e6, 1),
-                           "collide_us": round(k * 1e3, 2),
-                           "alg_GBs": round(38 * sb * case.cells / (k * 1e-3) / 1e9, 1)}
+                           "collide_us": round(k * 1e3, 2), "steps_per_launch": per,
+                           "alg_GBs": round(38 * sb * case.cells / (per * k * 1e-3) / 1e9, 1)}
             log(f"{name}: {forms[name]}")
         t = bench_v1(case, args.prec, fsteps, 5)
         forms["v1_abi_" + storage] = {"mlups": round(case.cells * fsteps / (t * 1e-3) / 1e6, 1),
@@ -368,7 +378,7 @@ def main():
         cpu = cpu_baseline(case, args.cpu_steps)
         log(f"cpu baseline {cpu['value']:.2f} MLUPS ({cpu['kind']}, {cpu['cores']} cores)")
     compact = info["nx"] == n + 2  # the engine chose compact rows
-    kernel = "collide_compact" if compact else "collide_fused"
+    kernel = "collide_pair" if per_launch == 2 else ("collide_compact" if compact else "collide_fused")
     traffic = load_traffic(workload, kernel)
     out = {
         "metric": METRIC,
@@ -385,15 +395,16 @@ def main():
         "data": "synthetic (analytic Taylor-Green initial state, no dataset)",
         "config": {"workload": workload, "grid": [n, n, n], "boundary": "periodic", "tau": 0.53, "U0": 0.05,
                    "path": "handle API: " + ("compact rows (nx = l + 2)" if compact else "rows padded to 128-byte "
-                                              "lines") + ", periodic boundary folded into the fused step",
+                                              "lines") + ", periodic boundary folded into the fused step"
+                   + (", two steps per launch" if per_launch == 2 else ""),
                    "layout_nx": info["nx"], "device_bytes": info["bytes"]},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "traffic_source": f"profiles/traffic.json: rocprofv3 FETCH_SIZE and WRITE_SIZE passes of this "
                                        f"kernel (profiles/{kernel}_taylor_green_256_fp32.md), not this run",
                      "traffic_over_alg": round(traffic / alg_bytes, 4) if traffic else None,
-                     "kernel": kernel, "kernel_avg_us": round(kern_avg_ms * 1e3, 2),
-                     "alg_bytes_per_launch": alg_bytes,
+                     "kernel": kernel, "kernel_avg_us": round(per_launch * kern_avg_ms * 1e3, 2),
+                     "steps_per_launch": per_launch, "alg_bytes_per_launch": alg_bytes,
                      "measured_copy_GBs": round(stream, 1) if stream else None,
                      "frac_of_measured_copy": round(achieved / stream, 4) if stream else None},
         "cpu_baseline": cpu,

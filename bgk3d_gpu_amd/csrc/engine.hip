@@ -342,7 +342,7 @@ int download_fields(bgk_handle& h, double* const (&outs)[4])
 namespace bgk {
 namespace eng {
 
-int handle_setup(bgk_handle& h, const bgk_config& c)
+int handle_setup(bgk_handle& h, const bgk_config& c, bool roomy)
 {
     if (c.l < 1 || c.m < 1 || c.n < 1) return fail(BGK_EINVAL, "grid %d x %d x %d", c.l, c.m, c.n);
     if (c.boundary < 0 || c.boundary > 3) return fail(BGK_EINVAL, "boundary %d", c.boundary);
@@ -389,8 +389,9 @@ int handle_setup(bgk_handle& h, const bgk_config& c)
     // start and end on lines (413 against 346 us per FP32 step at 256^3 over
     // compact rows).
     const double waste = (double)(round_up(c.l, h.A) - c.l) / (double)c.l;
-    h.pair = prefer_pair(c, round_up(c.l + 2, h.A) * h.ny, h.pgrid);
-    h.compact = c.layout == 2 || (c.layout == 0 && !h.pair && prefer_compact(c, waste));
+    const bool compact = c.layout == 2 || (c.layout == 0 && prefer_compact(c, waste));
+    h.pair = (roomy || !compact) && prefer_pair(c, round_up(c.l + 2, h.A) * h.ny, h.pgrid);
+    h.compact = compact && !h.pair;
     if (h.compact) {
         // cell (0, 1, k) of every population plane on a line start
         h.nx = c.l + 2;
@@ -481,7 +482,13 @@ int bgk_create(const bgk_config* cfg, bgk_handle** out)
     if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
         return cleanup(fail(BGK_EHIP, "stream creation failed"));
     void* region = nullptr;
-    if (hipMalloc(&region, lattice_bytes(*h)) != hipSuccess)
+    hipError_t got = hipMalloc(&region, lattice_bytes(*h));
+    if (got != hipSuccess && h->pair) {  // padded rows do not fit: compact ones may
+        (void)hipGetLastError();
+        handle_setup(*h, c, false);
+        got = hipMalloc(&region, lattice_bytes(*h));
+    }
+    if (got != hipSuccess)
         return cleanup(fail(BGK_ENOMEM, "cannot allocate %.2f GB of lattice", lattice_bytes(*h) / 1e9));
     place_lattices(*h, region);
     if (hipMemsetAsync(region, 0, lattice_bytes(*h), h->stream) != hipSuccess)

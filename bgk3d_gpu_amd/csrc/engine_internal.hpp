@@ -176,8 +176,10 @@ inline bool prefer_pair(const bgk_config& c, long plane, PairGrid& g)
 }
 
 // Validate `c` and fill the layout and the derived parameters of `h`
-// (no device call, no allocation).
-int handle_setup(bgk_handle& h, const bgk_config& c);
+// (no device call, no allocation).  `roomy`: two steps per launch also where
+// one step would run on compact rows, which need less memory than the padded
+// rows of collide_pair (130^3 FP32: 21 %).
+int handle_setup(bgk_handle& h, const bgk_config& c, bool roomy = true);
 
 // Device bytes of the two lattices of a handle set up by handle_setup.
 inline size_t lattice_bytes(const bgk_handle& h) { return (size_t)h.lstride * 2 * h.esize; }

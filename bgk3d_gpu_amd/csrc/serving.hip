@@ -191,6 +191,7 @@ struct Instance {
     int state = BGKS_QUEUED;
     bool has_mem = false;
     size_t off = 0, len = 0;
+    size_t roomy = 0;   // bytes with two steps per launch, where that takes more than len (else 0)
     int flag = -1;      // non-finite flag word while admitted
     int skipped = 0;    // chunks passed over in a row (queued or active)
     double diag[5] = {0, 0, 0, 0, 0};
@@ -450,6 +451,32 @@ int start(bgks_server& s, Instance& in, size_t off)
     return 0;
 }
 
+// Room for a request.  Its bytes are those of the smallest layout; it takes
+// the larger one of two steps per launch if every other queued request still
+// fits beside it.
+bool find_room(bgks_server& s, Instance& in, size_t& off)
+{
+    const size_t room = s.arena.size - s.arena.used();
+    if (in.roomy && in.roomy <= room) {
+        size_t left = room - in.roomy;
+        bool fits = true;
+        for (long long id : s.queue) {
+            const size_t len = id != in.id ? s.all.at(id)->len : 0;
+            fits = len <= left;
+            if (!fits) break;
+            left -= len;
+        }
+        if (fits && s.arena.alloc(in.roomy, off)) {
+            if (handle_setup(in.h, in.h.cfg) == 0) {
+                in.len = in.roomy;
+                return true;
+            }
+            s.arena.release(off, in.roomy);
+        }
+    }
+    return s.arena.alloc(in.len, off);
+}
+
 // Arrival order: the head of the queue waits for room.  Shortest first:
 // queued requests in order of their work, each admitted if it fits, except
 // that requests passed over kMaxSkips times come first, in arrival order,
@@ -461,7 +488,7 @@ int admit(bgks_server& s)
         while (!s.queue.empty() && !s.free_flags.empty()) {
             Instance& in = *s.all.at(s.queue.front());
             size_t off = 0;
-            if (!s.arena.alloc(in.len, off)) break;
+            if (!find_room(s, in, off)) break;
             if (int rc = start(s, in, off)) return rc;
             s.queue.pop_front();
         }
@@ -479,7 +506,7 @@ int admit(bgks_server& s)
         if (s.free_flags.empty()) break;
         Instance& in = *s.all.at(id);
         size_t off = 0;
-        if (!s.arena.alloc(in.len, off)) {
+        if (!find_room(s, in, off)) {
             if (in.skipped >= kMaxSkips) break;
             continue;
         }
@@ -543,7 +570,7 @@ int bgks_request_bytes(const bgks_request* r, size_t* bytes)
 {
     if (!r || !bytes) return fail(BGK_EINVAL, "null argument");
     bgk_handle h;
-    if (int rc = handle_setup(h, request_config(*r, 0))) return rc;
+    if (int rc = handle_setup(h, request_config(*r, 0), false)) return rc;
     *bytes = round_up((long)lattice_bytes(h), (long)kArenaAlign);
     return 0;
 }
@@ -638,12 +665,15 @@ int bgks_submit(bgks_server* s, const bgks_request* r, long long* id)
     if (r->steps < 0) return fail(BGK_EINVAL, "steps %lld", r->steps);
     if (r->rounding != 0 && r->rounding != 1) return fail(BGK_EINVAL, "rounding %d", r->rounding);
     auto in = std::make_unique<Instance>();
-    if (int rc = handle_setup(in->h, request_config(*r, s->device))) return rc;
+    if (int rc = handle_setup(in->h, request_config(*r, s->device), false)) return rc;
     in->h.borrowed = true;
     in->h.stream = s->stream;
     in->h.scratch = s->scratch;
     in->h.hscratch = s->hscratch;
     in->len = round_up((long)lattice_bytes(in->h), (long)kArenaAlign);
+    bgk_handle wide;
+    if (int rc = handle_setup(wide, in->h.cfg)) return rc;
+    if (wide.pair && !in->h.pair) in->roomy = round_up((long)lattice_bytes(wide), (long)kArenaAlign);
     if (in->len > s->arena.size)
         return fail(BGK_ENOMEM, "request needs %.3f GB, the budget is %.3f GB", in->len / 1e9, s->arena.size / 1e9);
     in->req = *r;

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import oracle_support as O
+from bgk3d_gpu_amd import serving as S
 from bgk3d_gpu_amd.cases import Case
 from bgk3d_gpu_amd.engine import Engine
 
@@ -103,4 +104,24 @@ def test_les_in_fp64_matches_single_steps(gpu, kw, storage, mixed):
                 eng.step(c)
             out.append(eng.populations())
     assert np.isfinite(out[0]).all() and np.any(out[0] != 0)
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n,storage", [(87, "f32"), (75, "f64")])
+def test_server_takes_the_layout_that_fits(gpu, n, storage):
+    """A served request whose two-step layout needs more bytes than
+    request_bytes: admitted into exactly that much with one step per launch,
+    into more with two, with the same populations."""
+    out = []
+    need = S.request_bytes(S.Request(n, 200.0, storage, 30))
+    for budget in (need, 3 * need):
+        srv = S.Server(budget, chunk_steps=7)
+        try:
+            rid = srv.submit(S.Request(n, 200.0, storage, 30, keep=True))
+            while rid not in srv.advance():
+                pass
+            out.append([srv.population(rid, d, n) for d in (0, 5, 18)])
+        finally:
+            srv.close()
+    assert np.isfinite(out[0]).all() and np.any(out[0][0] != 0)
     assert np.array_equal(out[0], out[1])
