@@ -10,9 +10,10 @@
 // The populations' z planes are interleaved (plane k of population d at
 // (19 k + d) planes from the start), so one step's reads and writes move
 // through two compact windows of the lattices instead of 37 separate
-// arrays.  Direction 19 is updated in place and lives only in lattice 0;
-// directions 1..18 alternate between the two lattices (the reference's
-// pointer swap, SRC/col_MC.F90:539-596), tracked by `cur`.
+// arrays.  Directions 1..18 alternate between the two lattices (the
+// reference's pointer swap, SRC/col_MC.F90:539-596), tracked by `cur`; so
+// does direction 19 in a launch of two steps (collide_pair), tracked by
+// `rest`, while a single step updates it in place.
 #include "engine_internal.hpp"
 
 #include <algorithm>

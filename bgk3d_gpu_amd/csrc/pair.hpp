@@ -19,7 +19,7 @@
 // The first step is taken twice for cells within one cell of a tile's border
 // (with 13 rows, 64 x 13 tiles: 16 waves for 13 rows, and 2 planes more per
 // block), their reads from L2: the tiles of one XCD are neighbours and walk up
-// together, and HBM is read 1.07 times (FETCH_SIZE, 256^3 FP32).
+// together, and HBM is read 1.09 times (FETCH_SIZE, 256^3 FP32).
 //
 // Measured at 256^3 FP32, us per step: 268 (410 with one step per launch), of
 // which arithmetic and exchange alone take 78, without the loads 136, without

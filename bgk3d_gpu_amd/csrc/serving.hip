@@ -9,8 +9,8 @@
 // budget; requests are admitted in arrival order while the arena can hold
 // them.  The requests of a chunk are split by (storage type, rounding, row
 // layout) group into sub-batches of at most 512 MB of lattices, and each
-// sub-batch runs all the chunk's steps, one launch per step, before the
-// next.  A request alone in its sub-batch runs the engine's own kernel; the
+// sub-batch runs all the chunk's steps, one launch per step or per two
+// (collide_pair, by the engine's rule), before the next.  A request alone in its sub-batch runs the engine's own kernel; the
 // launch grid of a larger sub-batch is the concatenation of its requests'
 // row blocks, and a block finds its request through a per-block owner table
 // and then runs the same per-cell code as the single-request kernel.  So a

@@ -6,7 +6,7 @@
  * 128-byte line), fold every boundary condition into the pull (no halo
  * kernels per step), store populations in FP32, FP64, FP16 or BF16 (shifted
  * f - w, collision in FP32 or FP64), and advance many independent solves
- * together, one launch per step for all of them (bgks_*).
+ * together, one launch per step or two for all of them (bgks_*).
  *
  * The reference has no such API: its driver owns the arrays and calls the
  * per-routine symbols of bgk3d_gpu.h (SRC/bgk3d.F90:169-196).  Each field
@@ -65,11 +65,14 @@ typedef struct bgk_config {
                              reference's expression order (the plain F16 form uses a leaner
                              FP32 arithmetic); 2 MIXED2: storage BGK_F32, collision in FP64 */
     int layout;           /* 0 choose, 1 rows padded to 128-byte lines, 2 compact rows of l + 2
-                             cells.  The default takes compact rows
+                             cells.  The default takes padded rows
+                             where two steps per launch run faster (FP32 and FP64 storage, from
+                             about 32^3 up), else compact rows
                              where they measured faster: when padding would leave more than 3 %
                              of a row unused in its last line (9 % with 16-bit storage; a line
                              holds 32 values in FP32, 16 in FP64, 64 in 16-bit storage), and
-                             with FP32/FP64 storage for lattices of 2^24 cells or more */
+                             with FP32/FP64 storage for lattices of 2^24 cells or more, or where
+                             the padded lattice cannot be allocated */
 } bgk_config;
 
 typedef struct bgk_handle bgk_handle;
@@ -86,8 +89,8 @@ int bgk_step(bgk_handle* h, int nsteps);
 int bgk_sync(bgk_handle* h);
 
 /* Run nsteps and time them: total wall time of the steps (hipEvents on the
- * handle's stream) and the mean duration of the fused collide kernel
- * (events bracketing each launch). */
+ * handle's stream) and the mean duration of the fused collide kernel per
+ * step (events bracketing each launch, which takes one step or two). */
 int bgk_time_steps(bgk_handle* h, int nsteps, double* total_ms, double* collide_avg_ms);
 
 /* Global means {<u>, <v>, <w>, <rho>, <0.5|u|^2>} (SRC/diagno.F90), FP64 sums. */
@@ -159,7 +162,7 @@ const char* bgk_last_error(void);
  * HBM budget) can hold their two lattices; the requests scheduled for a
  * chunk advance sub-batch by sub-batch (at most 512 MB of lattices of one
  * storage, rounding and row layout), one kernel launch per sub-batch and
- * step, on one stream; requests join and leave between chunks of at
+ * step or two steps, on one stream; requests join and leave between chunks of at
  * most chunk_steps steps, cut shorter by a chunk-time target if one is set
  * (see enum bgks_policy).  A request whose populations turn non-finite (the
  * step kernel checks every cell) is retired as unstable at the end of that
@@ -214,7 +217,9 @@ int bgks_set_chunk_time(bgks_server* s, double target_ms);
 int bgks_schedule(const long long* remaining, const long long* cells, const int* skipped, int count,
                   long long min_cells_per_step, int max_skips, int* selected, int* n_selected);
 
-/* Device bytes a request holds while admitted (both lattices, padded). */
+/* Device bytes a request needs while admitted (both lattices).  It holds up
+ * to a line per row more, for two steps per launch, while every queued
+ * request still fits beside it. */
 int bgks_request_bytes(const bgks_request* r, size_t* bytes);
 
 /* Queue a request; fails with BGK_ENOMEM if it can never fit the budget. */
