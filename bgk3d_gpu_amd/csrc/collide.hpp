@@ -71,10 +71,8 @@ struct FusedArgs {
     // Inflow velocity: compact rows under the inflow boundary write both x
     // faces from the halo lanes (compact_cells).
     C uin;
-    // Two steps in one pass (pair.hpp): direction 19 of the lattice written,
-    // and the second step's seed.
+    // Two steps in one pass (pair.hpp): direction 19 of the lattice written.
     S* brest;
-    uint32_t seed2;
 };
 
 // Raise the non-finite flag of p (if any) when the rest population v is not

@@ -236,7 +236,6 @@ FusedArgs<S> fused_args(const bgk_handle& h, int cur, int rest)
     else
         p.lend = h.cfg.boundary == BGK_BC_INFLOW ? 0 : (int)round_up(h.cfg.l, h.A);
     p.seed = step_seed(h.cfg.seed, h.steps);
-    p.seed2 = step_seed(h.cfg.seed, h.steps + 1);
     p.pstride = h.plane;
     p.uin = (C)h.u_inflow;
     return p;

@@ -16,7 +16,7 @@ void launch_fused(bgk_handle& h, bool pair)
     const FusedArgs<S> p = fused_args<S>(h, h.cur, h.rest);
     if constexpr (kPairs<S>) {
         if (pair) {
-            launch_pair<S, BX, BY, BZ, OB, FM, SR>(p, h.pgrid, h.stream);
+            launch_pair<S, BX, BY, BZ, OB, FM>(p, h.pgrid, h.stream);
             return;
         }
     }

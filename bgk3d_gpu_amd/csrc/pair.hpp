@@ -96,10 +96,6 @@ __device__ __forceinline__ uint32_t lane_offset(uint32_t v)
 template <size_t N>
 struct BitsOf;
 template <>
-struct BitsOf<2> {
-    typedef uint16_t type;
-};
-template <>
 struct BitsOf<4> {
     typedef uint32_t type;
 };
@@ -186,26 +182,12 @@ __device__ __forceinline__ void bgk_collide_shifted(const R (&x)[19], R omega, R
 
 // The step of one cell, rounded to the storage type, in the form the one-step
 // kernels use for S; each value goes to sink(d, value).
-template <typename S, int FMODE, int SR, typename Sink>
+template <typename S, int FMODE, typename Sink>
 __device__ __forceinline__ void pair_collide(const FusedArgs<S>& p, const typename Storage<S>::compute (&x)[19],
-                                             uint32_t seed, uint32_t cell, Sink&& sink)
+                                             Sink&& sink)
 {
-    typedef typename Storage<S>::compute C;
-    constexpr bool LES = (FMODE & 4) != 0;
-    uint32_t r = 0;
-    if (SR) r = hash32(seed ^ cell);
-    auto round = [&](auto dc, C v) {
-        constexpr int d = decltype(dc)::value;
-        sink(dc, Rounder<S, SR>::cvt(v, SR ? sr_word(r, d) : 0u));
-    };
-    if constexpr (Storage<S>::lean) {
-        C fx, fy, fz, o[19];
-        force_terms<C, (FMODE & 3)>(density_ref(x, p.cst.cte1), p.fgrad, p.fx, p.fy, p.fz, fx, fy, fz);
-        bgk_collide_lean<C, LES>(x, p.omega, fx, fy, fz, p.cst, o, p.cte_s);
-        for_each_dir([&](auto dc) { round(dc, o[decltype(dc)::value]); });
-    } else {
-        bgk_collide_shifted<C, (FMODE & 3), LES>(x, p.omega, p.fgrad, p.cte_s, round);
-    }
+    bgk_collide_shifted<typename Storage<S>::compute, (FMODE & 3), (FMODE & 4) != 0>(
+        x, p.omega, p.fgrad, p.cte_s, [&](auto dc, auto v) { sink(dc, Rounder<S, 0>::cvt(v, 0u)); });
 }
 
 // v where mask is all ones, +0 where it is 0 (a select of 19 values would be
@@ -215,19 +197,15 @@ __device__ __forceinline__ S masked(S v, uint32_t mask)
 {
     if constexpr (sizeof(S) == 8)
         return __builtin_bit_cast(S, __builtin_bit_cast(uint64_t, v) & ((uint64_t)mask << 32 | mask));
-    else if constexpr (sizeof(S) == 4)
-        return __builtin_bit_cast(S, __builtin_bit_cast(uint32_t, v) & mask);
     else
-        return __builtin_bit_cast(S, (uint16_t)(__builtin_bit_cast(uint16_t, v) & (uint16_t)mask));
+        return __builtin_bit_cast(S, __builtin_bit_cast(uint32_t, v) & mask);
 }
 
 // Stored bits of a value, as the loads of this kernel return them.
 template <typename S>
 __device__ __forceinline__ S load_raw(const S* p)
 {
-    if constexpr (sizeof(S) == 2)
-        return Storage<S>::raw(p);
-    else if constexpr (std::is_same<S, mix32_t>::value)
+    if constexpr (std::is_same<S, mix32_t>::value)
         return mix32_t{gmem(p)->v};
     else
         return *gmem(p);
@@ -252,10 +230,9 @@ constexpr bool kPairs = sizeof(S) >= 4;
 
 // Two steps of the tile of 64 / RW cells x th rows whose first cell is (x0, j0,
 // k0); with RW = 2 a wave holds two rows.  `lone`: the tile spans the row.
-// `seed`, `seed2`: the two steps' rounding seeds.
-template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, int SR, int RW>
+template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, int RW>
 __device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typename BitsOf<sizeof(S)>::type* lds, int x0,
-                                          int j0, int k0, int th, int zc, bool lone, uint32_t seed, uint32_t seed2)
+                                          int j0, int k0, int th, int zc, bool lone)
 {
     constexpr int TY = PairShape<S>::TY;
     constexpr bool DB = PairShape<S>::DB;
@@ -388,7 +365,7 @@ __device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typenam
             x[d] = Storage<S>::widen(raw[d]);
             if constexpr (BZ == AX_LID) x[d] = lid_value<S, d>(x[d], cz_of(d) < 0 && kk == p.n, p.lidforce);
         });
-        pair_collide<S, FMODE, SR>(p, x, seed, ref_cell(p, i, j, plane(kk)), [&](auto dc, S w) {
+        pair_collide<S, FMODE>(p, x, [&](auto dc, S w) {
             constexpr int d = decltype(dc)::value;
             v[d] = w;
             if constexpr (!stays(d) && BX != AX_HALO) buf[lds_slot(d) * POP + at] = __builtin_bit_cast(Bits, w);
@@ -496,7 +473,7 @@ __device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typenam
             char* moving = scalar_base(reinterpret_cast<char*>(p.b[0] + p.nxy * (kk - 1)));
             char* resting = scalar_base(reinterpret_cast<char*>(p.brest + p.nxy * (kk - 1)));
             const uint32_t off = lane_offset(to);
-            pair_collide<S, FMODE, SR>(p, x, seed2, ref_cell(p, i, j, kk - 1), [&](auto dc, S w) {
+            pair_collide<S, FMODE>(p, x, [&](auto dc, S w) {
                 constexpr int d = decltype(dc)::value;
                 char* base = d == 18 ? resting : moving + d * p.pstride * ES;
                 store_nt(reinterpret_cast<S*>(base + (uint64_t)off), masked(w, live));
@@ -546,9 +523,8 @@ __device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typenam
 }
 
 // Two steps of one tile of the launch.
-template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, int SR>
-__device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid& g, int tile, uint32_t seed,
-                                          uint32_t seed2)
+template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE>
+__device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid& g, int tile)
 {
     typedef typename BitsOf<sizeof(S)>::type Bits;
     __shared__ Bits lds_[(PairShape<S>::DB ? 2 : 1) * 16 * PairShape<S>::POP];
@@ -557,11 +533,11 @@ __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid&
     const int k0 = 1 + (tile / per) * g.zc;
     const bool lone = g.tx + (g.ty2 ? 1 : 0) == 1;
     if (q < g.tx * g.ty)
-        pair_rows<S, BX, BY, BZ, OBST, FMODE, SR, 1>(p, lds, 1 + q % g.tx * kTileX, 1 + q / g.tx * g.th, k0, g.th, g.zc,
-                                                     lone, seed, seed2);
+        pair_rows<S, BX, BY, BZ, OBST, FMODE, 1>(p, lds, 1 + q % g.tx * kTileX, 1 + q / g.tx * g.th, k0, g.th, g.zc,
+                                                 lone);
     else
-        pair_rows<S, BX, BY, BZ, OBST, FMODE, SR, 2>(p, lds, 1 + g.tx * kTileX, 1 + (q - g.tx * g.ty) * 2 * g.th, k0,
-                                                     2 * g.th, g.zc, lone, seed, seed2);
+        pair_rows<S, BX, BY, BZ, OBST, FMODE, 2>(p, lds, 1 + g.tx * kTileX, 1 + (q - g.tx * g.ty) * 2 * g.th, k0,
+                                                 2 * g.th, g.zc, lone);
 }
 
 // Block x of n blocks as the b-th tile: consecutive tiles on one XCD (blocks
@@ -572,11 +548,11 @@ __device__ __forceinline__ int xcd_tile(int x, int n)
     return (x >> 3) < per ? (x & 7) * per + (x >> 3) : n;
 }
 
-template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, int SR>
+template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE>
 __global__ __launch_bounds__(64 * (PairShape<S>::TY + 3)) void collide_pair(FusedArgs<S> p, PairGrid g)
 {
     const int tile = xcd_tile((int)blockIdx.x, g.total);
-    if (tile < g.total) pair_tile<S, BX, BY, BZ, OBST, FMODE, SR>(p, g, tile, p.seed, p.seed2);
+    if (tile < g.total) pair_tile<S, BX, BY, BZ, OBST, FMODE>(p, g, tile);
 }
 
 // Tiles of an l x m x n lattice with at most `rows` rows: the rows and planes
@@ -624,10 +600,10 @@ inline PairGrid pair_grid(int l, int m, int n, int rows, double& cost, double cu
 
 inline int pair_blocks(int tiles) { return ceil_div(tiles, 8) * 8; }
 
-template <typename S, int BX, int BY, int BZ, bool OB, int FM, int SR>
+template <typename S, int BX, int BY, int BZ, bool OB, int FM>
 void launch_pair(const FusedArgs<S>& p, const PairGrid& g, hipStream_t stream)
 {
-    hipLaunchKernelGGL((collide_pair<S, BX, BY, BZ, OB, FM, SR>), dim3((unsigned)pair_blocks(g.total)),
+    hipLaunchKernelGGL((collide_pair<S, BX, BY, BZ, OB, FM>), dim3((unsigned)pair_blocks(g.total)),
                        dim3(64 * (PairShape<S>::TY + 3)), 0, stream, p, g);
 }
 

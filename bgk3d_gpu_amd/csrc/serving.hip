@@ -128,7 +128,7 @@ __global__ __launch_bounds__(64 * (PairShape<S>::TY + 3)) void collide_pair_batc
     if (b >= n) return;
     const uint32_t tile = base + (uint32_t)b;
     const BatchSlot<S>& sl = slots[__builtin_amdgcn_readfirstlane((int)owner[tile])];
-    pair_tile<S, AX_WALL, AX_WALL, AX_LID, false, 0, 0>(sl.args[launch & 1], sl.pg, (int)(tile - sl.tile0), 0u, 0u);
+    pair_tile<S, AX_WALL, AX_WALL, AX_LID, false, 0>(sl.args[launch & 1], sl.pg, (int)(tile - sl.tile0));
 }
 
 double clock_now()
@@ -378,7 +378,7 @@ void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, int launch, 
         p.seed = step_seed(sl.cfg_seed, sl.steps0 + t);
         if constexpr (kPairs<S>) {
             if (pair) {
-                launch_pair<S, AX_WALL, AX_WALL, AX_LID, false, 0, SR>(p, sl.pg, stream);
+                launch_pair<S, AX_WALL, AX_WALL, AX_LID, false, 0>(p, sl.pg, stream);
                 return;
             }
         }
