@@ -71,7 +71,12 @@ Geometry geom(int l, int m, int n, int nx, int ny)
     return g;
 }
 
-constexpr int kFaceThreads = 256;
+// Threads per block of the halo kernels: one wave.  A face thread is a chain
+// of scattered loads and stores, so what counts on a small lattice is how many
+// CUs work: the 64^3 cavity's faces fill 384 blocks of 64 threads, 96 of 256
+// (per step 20.5 -> 15.8 us FP32, 32 -> 28 FP64; 256^3 and 400^3 Taylor-Green
+// and the 128^3 channel unchanged; 128 threads 17.5).
+constexpr int kFaceThreads = 64;
 
 // Host-side check of the caller's arguments before any kernel is launched on
 // them: positive sizes, rows and planes that hold the halo (nx >= l+2,
