@@ -646,8 +646,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FusedWaves<
 // cells of its output arrays: no routine reads them before the next boundary
 // call rewrites every halo value a pull uses.  A line the kernel writes only
 // in part costs the L2 a read of that line from HBM first: 484 against
-// 441 us per FP32 launch at 256^3.
-template <typename S, int FMODE, bool NT0, bool WL = false>
+// 441 us per FP32 launch at 256^3.  NT: streaming stores (v1_abi.hip).
+template <typename S, int FMODE, bool NT0, bool WL = false, bool NT = true>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FusedWaves<S, FMODE>::value))) void collide_flat(
     FusedArgs<S> p)
 {
@@ -676,13 +676,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FusedWaves<
     if constexpr (sizeof(S) == 8 && !LES) {
         bgk_collide_stream(x, p.omega, fx, fy, fz, p.cst, [&](auto dc, C v) {
             constexpr int d = decltype(dc)::value;
-            store_nt((d < 18 ? p.b[d] : p.a[18]) + (row + i), live ? v : C(0));
+            store_to<NT>((d < 18 ? p.b[d] : p.a[18]) + (row + i), live ? v : C(0));
         });
     } else {
         C o[19];
         bgk_collide_ref<C, LES>(x, p.omega, fx, fy, fz, p.cst, o, p.cte_s);
 #pragma unroll
-        for (int d = 0; d < 19; ++d) store_nt((d < 18 ? p.b[d] : p.a[18]) + (row + i), live ? o[d] : C(0));
+        for (int d = 0; d < 19; ++d) store_to<NT>((d < 18 ? p.b[d] : p.a[18]) + (row + i), live ? o[d] : C(0));
     }
 }
 

@@ -184,6 +184,15 @@ int handle_setup(bgk_handle& h, const bgk_config& c, bool roomy = true);
 // Device bytes of the two lattices of a handle set up by handle_setup.
 inline size_t lattice_bytes(const bgk_handle& h) { return (size_t)h.lstride * 2 * h.esize; }
 
+// Whether the lattices a launch works on, `bytes` together, are stored with
+// plain instead of streaming stores: the next step then finds them in the
+// 256 MB last-level cache.  Above that streaming is faster, and below 80 MB
+// too (FP32, two steps per launch, us per step, streaming against plain: 48^3
+// 5.7 / 6.2, 64^3 6.4 / 6.7, 80^3 15.0 / 12.0, 100^3 25.0 / 20.2, 112^3 30.4 / 23.4,
+// 128^3 (411 MB) 36.0 / 37.9; FP64 64^3 (106 MB) 10.7 / 10.8, 75^3 20.3 / 17.0,
+// 90^3 30.7 / 25.0, 100^3 (354 MB) 43.0 / 45.7).
+inline bool keep_in_cache(size_t bytes) { return bytes >= 80000000 && bytes <= size_t(1) << 28; }
+
 // Point mem[0] and mem[1] (the two lattices) into one region of
 // lattice_bytes(h) bytes.
 inline void place_lattices(bgk_handle& h, void* region)

@@ -230,7 +230,7 @@ constexpr bool kPairs = sizeof(S) >= 4;
 
 // Two steps of the tile of 64 / RW cells x th rows whose first cell is (x0, j0,
 // k0); with RW = 2 a wave holds two rows.  `lone`: the tile spans the row.
-template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, int RW>
+template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, bool NT, int RW>
 __device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typename BitsOf<sizeof(S)>::type* lds, int x0,
                                           int j0, int k0, int th, int zc, bool lone)
 {
@@ -476,7 +476,7 @@ __device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typenam
             pair_collide<S, FMODE>(p, x, [&](auto dc, S w) {
                 constexpr int d = decltype(dc)::value;
                 char* base = d == 18 ? resting : moving + d * p.pstride * ES;
-                store_nt(reinterpret_cast<S*>(base + (uint64_t)off), masked(w, live));
+                store_to<NT>(reinterpret_cast<S*>(base + (uint64_t)off), masked(w, live));
                 if constexpr (d == 18) flag_nonfinite(p, Storage<S>::widen(w));
             });
         }
@@ -523,7 +523,7 @@ __device__ __forceinline__ void pair_rows(const FusedArgs<S>& p, BGK_LDS typenam
 }
 
 // Two steps of one tile of the launch.
-template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE>
+template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, bool NT = true>
 __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid& g, int tile)
 {
     typedef typename BitsOf<sizeof(S)>::type Bits;
@@ -533,10 +533,10 @@ __device__ __forceinline__ void pair_tile(const FusedArgs<S>& p, const PairGrid&
     const int k0 = 1 + (tile / per) * g.zc;
     const bool lone = g.tx + (g.ty2 ? 1 : 0) == 1;
     if (q < g.tx * g.ty)
-        pair_rows<S, BX, BY, BZ, OBST, FMODE, 1>(p, lds, 1 + q % g.tx * kTileX, 1 + q / g.tx * g.th, k0, g.th, g.zc,
+        pair_rows<S, BX, BY, BZ, OBST, FMODE, NT, 1>(p, lds, 1 + q % g.tx * kTileX, 1 + q / g.tx * g.th, k0, g.th, g.zc,
                                                  lone);
     else
-        pair_rows<S, BX, BY, BZ, OBST, FMODE, 2>(p, lds, 1 + g.tx * kTileX, 1 + (q - g.tx * g.ty) * 2 * g.th, k0,
+        pair_rows<S, BX, BY, BZ, OBST, FMODE, NT, 2>(p, lds, 1 + g.tx * kTileX, 1 + (q - g.tx * g.ty) * 2 * g.th, k0,
                                                  2 * g.th, g.zc, lone);
 }
 
@@ -548,11 +548,11 @@ __device__ __forceinline__ int xcd_tile(int x, int n)
     return (x >> 3) < per ? (x & 7) * per + (x >> 3) : n;
 }
 
-template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE>
+template <typename S, int BX, int BY, int BZ, bool OBST, int FMODE, bool NT = true>
 __global__ __launch_bounds__(64 * (PairShape<S>::TY + 3)) void collide_pair(FusedArgs<S> p, PairGrid g)
 {
     const int tile = xcd_tile((int)blockIdx.x, g.total);
-    if (tile < g.total) pair_tile<S, BX, BY, BZ, OBST, FMODE>(p, g, tile);
+    if (tile < g.total) pair_tile<S, BX, BY, BZ, OBST, FMODE, NT>(p, g, tile);
 }
 
 // Tiles of an l x m x n lattice with at most `rows` rows: the rows and planes
@@ -600,10 +600,10 @@ inline PairGrid pair_grid(int l, int m, int n, int rows, double& cost, double cu
 
 inline int pair_blocks(int tiles) { return ceil_div(tiles, 8) * 8; }
 
-template <typename S, int BX, int BY, int BZ, bool OB, int FM>
+template <typename S, int BX, int BY, int BZ, bool OB, int FM, bool NT = true>
 void launch_pair(const FusedArgs<S>& p, const PairGrid& g, hipStream_t stream)
 {
-    hipLaunchKernelGGL((collide_pair<S, BX, BY, BZ, OB, FM>), dim3((unsigned)pair_blocks(g.total)),
+    hipLaunchKernelGGL((collide_pair<S, BX, BY, BZ, OB, FM, NT>), dim3((unsigned)pair_blocks(g.total)),
                        dim3(64 * (PairShape<S>::TY + 3)), 0, stream, p, g);
 }
 

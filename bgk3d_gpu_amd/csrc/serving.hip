@@ -8,7 +8,7 @@
 // whose two lattices live in one device arena sized by the caller's HBM
 // budget; requests are admitted in arrival order while the arena can hold
 // them.  The requests of a chunk are split by (storage type, rounding, row
-// layout) group into sub-batches of at most 512 MB of lattices, and each
+// layout) group into sub-batches of at most 256 MB of lattices, and each
 // sub-batch runs all the chunk's steps, one launch per step or per two
 // (collide_pair, by the engine's rule), before the next.  A request alone in its sub-batch runs the engine's own kernel; the
 // launch grid of a larger sub-batch is the concatenation of its requests'
@@ -56,15 +56,17 @@ constexpr int kServeWaves = 6;
 constexpr size_t kArenaAlign = 64 << 10;
 // A chunk runs its steps sub-batch by sub-batch: consecutive requests of a
 // storage group whose lattices add up to at most this many bytes (one larger
-// request forms its own), each sub-batch all K steps before the next.  The
-// fused kernel streams faster over a small working set, whose address
-// translations stay cached from one launch to the next (measured on the
-// 16-request cavity mix, FP32 part: 30.9k MLUPS with 512 MB sub-batches,
-// 28.1k with 3 GB).  Every request advances the chunk's steps in order, so
-// results do not depend on the grouping.  A request alone in its sub-batch
-// runs the engine's own kernel (no block-to-request lookup); batching in one
-// launch pays only for requests too small to fill the GPU by themselves.
-constexpr size_t kSubBatchBytes = size_t(1) << 29;
+// request forms its own), each sub-batch all K steps before the next: what
+// the 256 MB last-level cache holds (keep_in_cache; FP32 cavities of 98^3 and
+// 109^3 take 51 us per step together, 20 and 21 one after the other).  One
+// step per launch, too, streams faster over a small working set, whose address
+// translations stay cached from one launch to the next (16-request cavity mix,
+// FP32 part: 30.9k MLUPS with 512 MB sub-batches, 28.1k with 3 GB).  Every
+// request advances the chunk's steps in order, so results do not depend on
+// the grouping.  A request alone in its sub-batch runs the engine's own kernel
+// (no block-to-request lookup); batching in one launch pays only for requests
+// too small to fill the GPU by themselves.
+constexpr size_t kSubBatchBytes = size_t(1) << 28;
 // Requests admitted at once: each holds one non-finite flag word.
 constexpr int kMaxFlags = 4096;
 // Shortest-first aging: chunks a request may be passed over in a row.
@@ -120,7 +122,7 @@ collide_batched_compact(const BatchSlot<S>* __restrict__ slots, const uint32_t* 
 
 // Two steps of every request of a sub-batch (collide_pair's tiles): the n
 // tiles from `base` on, owner[] the request of each.
-template <typename S>
+template <typename S, bool NT>
 __global__ __launch_bounds__(64 * (PairShape<S>::TY + 3)) void collide_pair_batched(
     const BatchSlot<S>* __restrict__ slots, const uint32_t* __restrict__ owner, uint32_t base, int n, int launch)
 {
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(64 * (PairShape<S>::TY + 3)) void collide_pair_batc
     if (b >= n) return;
     const uint32_t tile = base + (uint32_t)b;
     const BatchSlot<S>& sl = slots[__builtin_amdgcn_readfirstlane((int)owner[tile])];
-    pair_tile<S, AX_WALL, AX_WALL, AX_LID, false, 0>(sl.args[launch & 1], sl.pg, (int)(tile - sl.tile0));
+    pair_tile<S, AX_WALL, AX_WALL, AX_LID, false, 0, NT>(sl.args[launch & 1], sl.pg, (int)(tile - sl.tile0));
 }
 
 double clock_now()
@@ -287,6 +289,7 @@ struct SubBatch {
     uint32_t block0, nblocks;
     uint32_t tile0, ntiles;  // two-step launches
     int single;              // the member that is alone in this sub-batch, else -1
+    size_t bytes;            // lattices of its members
 };
 
 template <typename S>
@@ -302,12 +305,13 @@ int prepare_group(bgks_server& s, bgks_server::Group& g, const std::vector<Insta
     for (size_t q = 0; q < members.size(); ++q) {
         bgk_handle& h = members[q]->h;
         if (subs.empty() || (sub_bytes > 0 && sub_bytes + members[q]->len > kSubBatchBytes)) {
-            subs.push_back({total, 0, 0, 0, (int)q});
+            subs.push_back({total, 0, 0, 0, (int)q, 0});
             sub_bytes = 0;
         } else {
             subs.back().single = -1;
         }
         sub_bytes += members[q]->len;
+        subs.back().bytes = sub_bytes;
         sub_of[q] = subs.size() - 1;
         BatchSlot<S>& sl = slots[q];
         sl.args[0] = fused_args<S>(h, h.cur, h.rest);
@@ -378,7 +382,10 @@ void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, int launch, 
         p.seed = step_seed(sl.cfg_seed, sl.steps0 + t);
         if constexpr (kPairs<S>) {
             if (pair) {
-                launch_pair<S, AX_WALL, AX_WALL, AX_LID, false, 0>(p, sl.pg, stream);
+                if (keep_in_cache(sb.bytes))
+                    launch_pair<S, AX_WALL, AX_WALL, AX_LID, false, 0, false>(p, sl.pg, stream);
+                else
+                    launch_pair<S, AX_WALL, AX_WALL, AX_LID, false, 0, true>(p, sl.pg, stream);
                 return;
             }
         }
@@ -402,9 +409,15 @@ void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, int launch, 
     }
     if constexpr (kPairs<S>) {
         if (pair) {
-            hipLaunchKernelGGL((collide_pair_batched<S>), dim3((unsigned)pair_blocks((int)sb.ntiles)),
-                               dim3(64 * (PairShape<S>::TY + 3)), 0, stream, d_slots, g.d_owner, sb.tile0,
-                               (int)sb.ntiles, launch);
+            auto run = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)pair_blocks((int)sb.ntiles)),
+                                   dim3(64 * (PairShape<S>::TY + 3)), 0, stream, d_slots, g.d_owner, sb.tile0,
+                                   (int)sb.ntiles, launch);
+            };
+            if (keep_in_cache(sb.bytes))
+                run(collide_pair_batched<S, false>);
+            else
+                run(collide_pair_batched<S, true>);
             return;
         }
     }

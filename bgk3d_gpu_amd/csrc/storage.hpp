@@ -253,4 +253,15 @@ __device__ __forceinline__ void store_nt<f16r_t>(f16r_t* p, f16r_t v)
     __builtin_nontemporal_store(v.v, &gmem(p)->v);
 }
 
+// Streaming store, or a plain one where the lattices stay in the last-level
+// cache (keep_in_cache).
+template <bool NT, typename S>
+__device__ __forceinline__ void store_to(S* p, S v)
+{
+    if constexpr (NT)
+        store_nt(p, v);
+    else
+        store_value(p, v);
+}
+
 }  // namespace bgk

@@ -160,7 +160,7 @@ const char* bgk_last_error(void);
  *
  * Requests are admitted while the device arena reserved by bgks_create (the
  * HBM budget) can hold their two lattices; the requests scheduled for a
- * chunk advance sub-batch by sub-batch (at most 512 MB of lattices of one
+ * chunk advance sub-batch by sub-batch (at most 256 MB of lattices of one
  * storage, rounding and row layout), one kernel launch per sub-batch and
  * step or two steps, on one stream; requests join and leave between chunks of at
  * most chunk_steps steps, cut shorter by a chunk-time target if one is set

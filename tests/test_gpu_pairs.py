@@ -125,3 +125,21 @@ def test_server_takes_the_layout_that_fits(gpu, n, storage):
             srv.close()
     assert np.isfinite(out[0]).all() and np.any(out[0][0] != 0)
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("size,storage", [((64, 60, 60), "f32"), ((80, 80, 80), "f32"), ((112, 112, 112), "f32"),
+                                          ((90, 90, 90), "f64")], ids=["stream", "low", "high", "f64"])
+@pytest.mark.parametrize("name", ["ldc", "periodic", "inflow"])
+def test_stores_that_stay_in_cache(gpu, size, storage, name):
+    """Plain stores where both lattices fit the last-level cache (80 ... 256 MB),
+    against single steps, which always stream."""
+    case = Case(l=size[0], m=size[1], n=size[2], **CASES[name])
+    print(f"[gpu] cached stores {name} {storage} {size}", flush=True)
+    out = []
+    for chunks in ((4,), (1,) * 4):
+        with Engine(case, storage, layout=1) as eng:
+            for c in chunks:
+                eng.step(c)
+            out.append([eng.population(d) for d in (0, 5, 10, 18)])
+    assert np.isfinite(out[0]).all() and np.any(out[0][0] != 0)
+    assert np.array_equal(out[0], out[1])
