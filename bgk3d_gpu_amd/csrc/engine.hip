@@ -23,6 +23,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -287,6 +288,9 @@ int download_fields(bgk_handle& h, double* const (&outs)[4])
     const int workers = std::min(chunks, std::min(8, cpus));
     const size_t slot = (size_t)chunk * fields;  // values of one chunk
     const size_t bytes = slot * workers * sizeof(C);
+    // Threads may ask one handle for its fields at the same time: the staging
+    // belongs to one of them until its copies are done.
+    const std::lock_guard<std::mutex> lock(h.stage_lock);
     if (h.stage_bytes < bytes) {
         if (h.stage) (void)hipFree(h.stage);
         if (h.hstage) (void)hipHostFree(h.hstage);

@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -54,7 +55,9 @@ struct bgk_handle {
     int8_t* omask = nullptr;
     double* scratch = nullptr;
     double* hscratch = nullptr;
-    // device and pinned host staging of bgk_fields, from its first call on
+    // device and pinned host staging of bgk_fields, from its first call on;
+    // one call at a time uses (and may replace) it
+    std::mutex stage_lock;
     void *stage = nullptr, *hstage = nullptr;
     size_t stage_bytes = 0;
     long long steps = 0;
