@@ -305,6 +305,7 @@ int download_fields(bgk_handle& h, double* const (&outs)[4])
     std::atomic<int> next{0}, bad{0};
     auto work = [&](int w) {
         hipEvent_t done = nullptr;
+        (void)hipGetLastError();  // what an earlier call of this thread left is not this launch's
         bool ok = hipSetDevice(h.cfg.device) == hipSuccess &&
                   hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess;
         C *d = dev + slot * w, *p = host + slot * w;

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from bgk3d_gpu_amd import engine as E
+from bgk3d_gpu_amd import runtime as rt
 from bgk3d_gpu_amd.cases import Case
 from bgk3d_gpu_amd.engine import Engine
 
@@ -36,3 +37,14 @@ def test_fields_from_several_threads(gpu):
         for t in threads:
             t.join()
         assert not wrong, (wrong[:4], E.lib().bgk_last_error())
+
+
+def test_fields_after_a_refused_handle(gpu):
+    """A lattice that cannot be allocated (17 TB) leaves the other handles of
+    the thread as they were."""
+    with Engine(Case("ldc", 20, 20, 20, svisc=0.05, u0=0.1), "f32") as eng:
+        eng.step(2)
+        want = eng.fields()
+        with pytest.raises(rt.BGKError):
+            Engine(Case("ldc", 4000, 4000, 4000, svisc=0.05, u0=0.1), "f64")
+        assert np.array_equal(eng.fields(), want)
