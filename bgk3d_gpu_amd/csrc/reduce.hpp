@@ -125,20 +125,26 @@ __global__ __launch_bounds__(kRedThreads) void diagno_partial(Lattice19<S> a, Ge
     }
 }
 
+// Rows whose varm sums are held at a time (32 bytes each, 8 MB): longer
+// lattices take several passes of whole planes.
+constexpr long kVarmRows = 1L << 18;
+inline int varm_planes(int m, int n) { return kVarmRows / m >= n ? n : (kVarmRows > m ? (int)(kVarmRows / m) : 1); }
+
 // varm (SRC/varm.F90:56-92), first pass: the sums of u, w (y velocity), v (z
-// velocity) and the density over each row (j, k), part[4 * row + {0,1,2,3}],
-// row = (j - 1) + m (k - 1).  A wave per row, so the lattice is read once with
-// the whole GPU at work (a block per plane left 106 of 256 CUs idle at 150
-// planes, and the planes along j were a second read).
+// velocity) and the density over each row (j, k) of the `planes` planes from
+// k = k0 + 1 on, part[4 * row + {0,1,2,3}], row = (j - 1) + m (k - 1 - k0).  A
+// wave per row, so the lattice is read once with the whole GPU at work (a
+// block per plane left 106 of 256 CUs idle at 150 planes, and the planes
+// along j were a second read).
 template <typename S>
 __global__ __launch_bounds__(kRedThreads) void varm_rows(Lattice19<S> a, Geometry g, typename Storage<S>::compute cte1,
-                                                         double* __restrict__ part)
+                                                         int k0, int planes, double* __restrict__ part)
 {
     typedef typename Storage<S>::compute R;
     const int lane = threadIdx.x & 63;
     const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= (long)g.m * g.n) return;
-    const int j = 1 + (int)(r % g.m), k = 1 + (int)(r / g.m);
+    if (r >= (long)g.m * planes) return;
+    const int j = 1 + (int)(r % g.m), k = 1 + k0 + (int)(r / g.m);
     double v[4] = {0, 0, 0, 0};
     for (int i = 1 + lane; i <= g.l; i += 64) {
         R x[19];
@@ -158,29 +164,30 @@ __global__ __launch_bounds__(kRedThreads) void varm_rows(Lattice19<S> a, Geometr
     }
 }
 
-// Second pass: blocks 0..n-1 fold the velocities of plane k = block + 1 into
-// out[3 * block + {0,1,2}], blocks n..n+m-1 the densities of plane j into
-// out[3 * n + block - n].  `out` as in fold_partials.
-static __global__ __launch_bounds__(kRedThreads) void varm_fold(const double* __restrict__ part, int m, int n,
-                                                         double* __restrict__ out)
+// Second pass: blocks 0..planes-1 fold the velocities of plane k = k0 + 1 +
+// block into out[3 * (k - 1) + {0,1,2}], the next m blocks the densities of
+// plane j into out[3 * n + j - 1], on top of those of the planes below k0.
+// `out` as in fold_partials.
+static __global__ __launch_bounds__(kRedThreads) void varm_fold(const double* __restrict__ part, int m, int n, int k0,
+                                                                int planes, double* __restrict__ out)
 {
-    const int b = (int)blockIdx.x;
+    const int b = (int)blockIdx.x, j0 = b - planes;
     double v[3] = {0, 0, 0};
-    if (b < n) {
+    if (j0 < 0) {
         for (int j = threadIdx.x; j < m; j += kRedThreads) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) v[q] += part[4 * ((long)b * m + j) + q];
         }
     } else {
-        for (int k = threadIdx.x; k < n; k += kRedThreads) v[0] += part[4 * ((long)k * m + (b - n)) + 3];
+        for (int k = threadIdx.x; k < planes; k += kRedThreads) v[0] += part[4 * ((long)k * m + j0) + 3];
     }
     block_sum<3>(v);
     if (threadIdx.x == 0) {
-        if (b < n) {
+        if (j0 < 0) {
 #pragma unroll
-            for (int q = 0; q < 3; ++q) out[3 * b + q] = v[q];
+            for (int q = 0; q < 3; ++q) out[3 * (long)(k0 + b) + q] = v[q];
         } else {
-            out[3 * n + b - n] = v[0];
+            out[3 * (long)n + j0] = k0 ? out[3 * (long)n + j0] + v[0] : v[0];
         }
     }
 }
