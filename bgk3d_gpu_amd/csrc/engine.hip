@@ -111,6 +111,32 @@ __global__ void outflow_halo(Lattice19<S> a, Geometry g, bool refill, typename S
     }
 }
 
+// Direction 19 of one lattice into the other's place for it: `planes` z
+// levels, `plane` values each, nxy apart.
+template <typename S>
+__global__ void move_rest(const S* __restrict__ from, S* __restrict__ to, long plane, long nxy, int planes)
+{
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= plane * planes) return;
+    const long e = t % plane + t / plane * nxy;
+    to[e] = from[e];
+}
+
+// A whole lattice into other rows: interior cells from `from`, zeros in the
+// halo and in the row padding, which no folded boundary reads (planes of
+// `plane` values, the halo ones among them).
+template <typename S>
+__global__ void move_rows(Lattice19<S> from, Geometry gf, Lattice19<S> to, Geometry gt, long plane)
+{
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= plane * (gt.n + 2)) return;
+    const int k = (int)(t / plane), e = (int)(t % plane), j = e / gt.nx, i = e - j * gt.nx;
+    const bool inside = i >= 1 && i <= gt.l && j >= 1 && j <= gt.m && k >= 1 && k <= gt.n;
+    const long at = e + gt.nxy * k, src = inside ? gidx(gf, i, j, k) : 0;
+#pragma unroll
+    for (int d = 0; d < 19; ++d) to.p[d][at] = inside ? from.p[d][src] : S{};
+}
+
 // Momentum exchange over fluid cells of [is..ie]x[js..je]x[ks..ke]
 // (SRC/draglift.F90:77-176); the solid mask is held for a box around the
 // obstacle only (cells outside it are fluid).
@@ -173,6 +199,18 @@ bool sphere_solid(const bgk_handle& h, int i, int j, int k)
 
 int wrap(int v, int n) { return v < 1 ? v + n : (v > n ? v - n : v); }
 
+// The inflow face x = 0 of both lattices.
+template <typename S>
+void fill_inflow(bgk_handle& h)
+{
+    for (int buf = 0; buf < 2; ++buf) {
+        Lattice19<S> L;
+        for (int d = 0; d < 19; ++d) L.p[d] = h.arr<S>(buf, d);
+        hipLaunchKernelGGL(inflow_halo<S>, dim3(ceil_div((long)(h.cfg.m + 2) * (h.cfg.n + 2), 256)), dim3(256), 0,
+                           h.stream, L, h.geom(), (typename Storage<S>::compute)h.u_inflow);
+    }
+}
+
 template <typename S>
 int upload_state(bgk_handle& h)
 {
@@ -193,12 +231,7 @@ int upload_state(bgk_handle& h)
         return fail(BGK_EINVAL, "init mode %d not supported", c.init);
     }
     if (c.boundary == BGK_BC_INFLOW) {
-        for (int buf = 0; buf < 2; ++buf) {
-            Lattice19<S> L;
-            for (int d = 0; d < 19; ++d) L.p[d] = h.arr<S>(d == 18 ? 0 : buf, d);
-            hipLaunchKernelGGL(inflow_halo<S>, dim3(ceil_div((long)(c.m + 2) * (c.n + 2), 256)), dim3(256), 0,
-                               h.stream, L, h.geom(), (C)h.u_inflow);
-        }
+        fill_inflow<S>(h);
         ENG_HIP(hipStreamSynchronize(h.stream));
     }
     return 0;
@@ -397,19 +430,8 @@ int handle_setup(bgk_handle& h, const bgk_config& c, bool roomy)
     const double waste = (double)(round_up(c.l, h.A) - c.l) / (double)c.l;
     const bool compact = c.layout == 2 || (c.layout == 0 && prefer_compact(c, waste));
     h.pair = (roomy || !compact) && prefer_pair(c, round_up(c.l + 2, h.A) * h.ny, h.pgrid);
-    h.compact = compact && !h.pair;
-    if (h.compact) {
-        // cell (0, 1, k) of every population plane on a line start
-        h.nx = c.l + 2;
-        h.plane = round_up((long)h.nx * h.ny, h.A);
-        h.base = (h.A - h.nx % h.A) % h.A;
-    } else {
-        // cell (1, j, k) on a line start
-        h.nx = (int)round_up(c.l + 2, h.A);
-        h.plane = (long)h.nx * h.ny;
-        h.base = h.A - 1;
-    }
-    h.nxy = 19 * h.plane;
+    h.flex = h.pair && compact;
+    set_rows(h, compact && !h.pair);
     h.lstride = round_up(h.A + h.nxy * h.nz, h.A);
     // derived parameters in the collision kind (SRC/hencol.F90:31, :52;
     // SRC/bcond.driven.F90:61; SRC/build.bcond.F90:29-35)
@@ -431,6 +453,43 @@ int handle_setup(bgk_handle& h, const bgk_config& c, bool roomy)
     h.cte_s = c.cte_s < 0 ? (double)0.1f : K(c.cte_s);
 
     return 0;
+}
+
+int join_rest(bgk_handle& h)
+{
+    if (h.rest == h.cur) return 0;
+    by_storage(h.cfg, [&](auto tag) {
+        typedef decltype(tag) S;
+        hipLaunchKernelGGL(move_rest<S>, dim3(ceil_div(h.plane * h.nz, 256)), dim3(256), 0, h.stream,
+                           h.arr<S>(h.rest, 18), h.arr<S>(h.cur, 18), h.plane, h.nxy, h.nz);
+        return 0;
+    });
+    h.rest = h.cur;
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : fail(BGK_EHIP, "direction 19: %s", hipGetErrorString(e));
+}
+
+// The populations go to the other lattice, the one they leave is cleared: a
+// step's worth of reads and writes, and half of one more.
+int relayout(bgk_handle& h, bool compact)
+{
+    if (h.compact == compact) return 0;
+    if (int rc = join_rest(h)) return rc;
+    return by_storage(h.cfg, [&](auto tag) {
+        typedef decltype(tag) S;
+        const Lattice19<S> from = h.current<S>();
+        const Geometry gf = h.geom();
+        const int left = h.cur;
+        h.cur = h.rest = 1 - left;
+        set_rows(h, compact);
+        hipLaunchKernelGGL(move_rows<S>, dim3(ceil_div(h.plane * h.nz, 256)), dim3(256), 0, h.stream, from, gf,
+                           h.current<S>(), h.geom(), h.plane);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail(BGK_EHIP, "rows: %s", hipGetErrorString(e));
+        ENG_HIP(hipMemsetAsync(h.mem[left], 0, (size_t)h.lstride * h.esize, h.stream));
+        if (h.cfg.boundary == BGK_BC_INFLOW) fill_inflow<S>(h);
+        return 0;
+    });
 }
 
 }  // namespace eng
@@ -863,14 +922,7 @@ int bgk_restore_raw(bgk_handle* h, const char* path, int* itime)
     // the engine's own constant inflow face (both lattices)
     if (c.boundary == BGK_BC_INFLOW) {
         rc = by_storage(c, [&](auto tag) {
-            typedef decltype(tag) S;
-            typedef typename Storage<S>::compute C;
-            for (int buf = 0; buf < 2; ++buf) {
-                Lattice19<S> L;
-                for (int d = 0; d < 19; ++d) L.p[d] = d == 18 ? h->arr<S>(0, 18) : h->arr<S>(buf, d);
-                hipLaunchKernelGGL(inflow_halo<S>, dim3(ceil_div((long)(c.m + 2) * (c.n + 2), 256)), dim3(256), 0,
-                                   h->stream, L, h->geom(), (C)h->u_inflow);
-            }
+            fill_inflow<decltype(tag)>(*h);
             return hipStreamSynchronize(h->stream) == hipSuccess ? 0 : fail(BGK_EHIP, "inflow face");
         });
         if (rc) return rc;

@@ -38,8 +38,10 @@ struct bgk_handle {
     // compact layout: rows of l + 2 cells (collide_compact), else rows padded
     // to whole lines (collide_fused)
     bool compact = false;
-    // two steps per launch (collide_pair) where two are left, in tiles pgrid
-    bool pair = false;
+    // two steps per launch (collide_pair) where two are left, in tiles pgrid.
+    // `flex`: one step at a time would run on compact rows; lstride holds a
+    // lattice of either rows (relayout)
+    bool pair = false, flex = false;
     bgk::PairGrid pgrid{};
     void* mem[2] = {nullptr, nullptr};
     size_t bytes = 0;
@@ -183,6 +185,29 @@ inline bool prefer_pair(const bgk_config& c, long plane, PairGrid& g)
 // one step would run on compact rows, which need less memory than the padded
 // rows of collide_pair (130^3 FP32: 21 %).
 int handle_setup(bgk_handle& h, const bgk_config& c, bool roomy = true);
+
+// Rows of the handle from here on: compact, or padded to whole lines.
+inline void set_rows(bgk_handle& h, bool compact)
+{
+    h.compact = compact;
+    if (compact) {
+        // cell (0, 1, k) of every population plane on a line start
+        h.nx = h.cfg.l + 2;
+        h.plane = round_up((long)h.nx * h.ny, h.A);
+        h.base = (h.A - h.nx % h.A) % h.A;
+    } else {
+        // cell (1, j, k) on a line start
+        h.nx = (int)round_up(h.cfg.l + 2, h.A);
+        h.plane = (long)h.nx * h.ny;
+        h.base = h.A - 1;
+    }
+    h.nxy = 19 * h.plane;
+}
+
+// Queue the move of a flex handle's populations to the other rows, and of
+// direction 19 to the lattice of the others (relayout does that too).
+int relayout(bgk_handle& h, bool compact);
+int join_rest(bgk_handle& h);
 
 // Device bytes of the two lattices of a handle set up by handle_setup.
 inline size_t lattice_bytes(const bgk_handle& h) { return (size_t)h.lstride * 2 * h.esize; }

@@ -192,8 +192,9 @@ struct Instance {
     bgk_handle h;
     int state = BGKS_QUEUED;
     bool has_mem = false;
-    size_t off = 0, len = 0;
-    size_t roomy = 0;   // bytes with two steps per launch, where that takes more than len (else 0)
+    size_t off = 0, len = 0;  // its range of the arena, while has_mem
+    size_t need = 0;    // bytes of the smallest layout (request_bytes)
+    size_t roomy = 0;   // bytes with two steps per launch, where that takes more (else 0)
     int flag = -1;      // non-finite flag word while admitted
     int skipped = 0;    // chunks passed over in a row (queued or active)
     double diag[5] = {0, 0, 0, 0, 0};
@@ -464,30 +465,77 @@ int start(bgks_server& s, Instance& in, size_t off)
     return 0;
 }
 
-// Room for a request.  Its bytes are those of the smallest layout; it takes
-// the larger one of two steps per launch if every other queued request still
-// fits beside it.
-bool find_room(bgks_server& s, Instance& in, size_t& off)
+// All held lattices in their smallest layout, one after the other from the
+// arena's start on, in the order they lie in: what is free is one range.  A
+// lattice moves down, so its populations may have to step aside to its upper
+// half first.
+int gather(bgks_server& s)
 {
+    std::vector<Instance*> held;
+    for (auto& kv : s.all)
+        if (kv.second->has_mem) held.push_back(kv.second.get());
+    std::sort(held.begin(), held.end(), [](const Instance* x, const Instance* y) { return x->off < y->off; });
+    size_t at = 0;
+    for (Instance* in : held) {
+        bgk_handle& h = in->h;
+        if (int rc = in->len != in->need ? relayout(h, true) : join_rest(h)) return rc;
+        if (int rc = handle_setup(h, h.cfg, false)) return rc;
+        char* const to = static_cast<char*>(s.arena_mem) + at;
+        char* from = static_cast<char*>(h.mem[h.cur]);
+        const size_t bytes = (size_t)h.lstride * h.esize;
+        if (from != to && from < to + bytes) {
+            ENG_HIP(hipMemcpyAsync(h.mem[1], from, bytes, hipMemcpyDeviceToDevice, s.stream));
+            from = static_cast<char*>(h.mem[1]);
+        }
+        if (from != to) ENG_HIP(hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, s.stream));
+        place_lattices(h, to);
+        h.cur = h.rest = 0;
+        ENG_HIP(hipMemsetAsync(h.mem[1], 0, bytes, s.stream));
+        in->off = at;
+        in->len = in->need;
+        at += in->len;
+    }
+    s.arena.reset(s.arena.size);
+    size_t off;
+    if (at) s.arena.alloc(at, off);
+    return 0;
+}
+
+// Room for a request, `found` if there is.  It takes the larger layout of two
+// steps per launch if every other queued request still fits beside it.  A
+// later request must not wait for that, nor for the holes between the others
+// (one that was kept may hold its lattice for good): where the smallest
+// layouts of all leave enough, they are gathered.
+int find_room(bgks_server& s, Instance& in, size_t& off, bool& found)
+{
+    found = true;
     const size_t room = s.arena.size - s.arena.used();
     if (in.roomy && in.roomy <= room) {
         size_t left = room - in.roomy;
         bool fits = true;
         for (long long id : s.queue) {
-            const size_t len = id != in.id ? s.all.at(id)->len : 0;
-            fits = len <= left;
+            const size_t need = id != in.id ? s.all.at(id)->need : 0;
+            fits = need <= left;
             if (!fits) break;
-            left -= len;
+            left -= need;
         }
         if (fits && s.arena.alloc(in.roomy, off)) {
-            if (handle_setup(in.h, in.h.cfg) == 0) {
-                in.len = in.roomy;
-                return true;
-            }
-            s.arena.release(off, in.roomy);
+            if (int rc = handle_setup(in.h, in.h.cfg)) return rc;
+            in.len = in.roomy;
+            return 0;
         }
     }
-    return s.arena.alloc(in.len, off);
+    in.len = in.need;
+    if (s.arena.alloc(in.need, off)) return 0;
+    size_t held = 0;
+    for (auto& kv : s.all)
+        if (kv.second->has_mem) held += kv.second->need;
+    found = s.arena.size - held >= in.need;
+    if (found) {
+        if (int rc = gather(s)) return rc;
+        found = s.arena.alloc(in.need, off);
+    }
+    return 0;
 }
 
 // Arrival order: the head of the queue waits for room.  Shortest first:
@@ -501,7 +549,9 @@ int admit(bgks_server& s)
         while (!s.queue.empty() && !s.free_flags.empty()) {
             Instance& in = *s.all.at(s.queue.front());
             size_t off = 0;
-            if (!find_room(s, in, off)) break;
+            bool found = false;
+            if (int rc = find_room(s, in, off, found)) return rc;
+            if (!found) break;
             if (int rc = start(s, in, off)) return rc;
             s.queue.pop_front();
         }
@@ -519,7 +569,9 @@ int admit(bgks_server& s)
         if (s.free_flags.empty()) break;
         Instance& in = *s.all.at(id);
         size_t off = 0;
-        if (!find_room(s, in, off)) {
+        bool found = false;
+        if (int rc = find_room(s, in, off, found)) return rc;
+        if (!found) {
             if (in.skipped >= kMaxSkips) break;
             continue;
         }
@@ -683,12 +735,12 @@ int bgks_submit(bgks_server* s, const bgks_request* r, long long* id)
     in->h.stream = s->stream;
     in->h.scratch = s->scratch;
     in->h.hscratch = s->hscratch;
-    in->len = round_up((long)lattice_bytes(in->h), (long)kArenaAlign);
+    in->need = round_up((long)lattice_bytes(in->h), (long)kArenaAlign);
     bgk_handle wide;
     if (int rc = handle_setup(wide, in->h.cfg)) return rc;
     if (wide.pair && !in->h.pair) in->roomy = round_up((long)lattice_bytes(wide), (long)kArenaAlign);
-    if (in->len > s->arena.size)
-        return fail(BGK_ENOMEM, "request needs %.3f GB, the budget is %.3f GB", in->len / 1e9, s->arena.size / 1e9);
+    if (in->need > s->arena.size)
+        return fail(BGK_ENOMEM, "request needs %.3f GB, the budget is %.3f GB", in->need / 1e9, s->arena.size / 1e9);
     in->req = *r;
     in->id = s->next_id++;
     in->t_submit = clock_now();

@@ -219,7 +219,9 @@ int bgks_schedule(const long long* remaining, const long long* cells, const int*
 
 /* Device bytes a request needs while admitted (both lattices).  It holds up
  * to a line per row more, for two steps per launch, while every queued
- * request still fits beside it. */
+ * request still fits beside it; a request that comes later and does not fit
+ * takes that room back (the lattices, of finished requests that are kept too,
+ * move to the arena's start). */
 int bgks_request_bytes(const bgks_request* r, size_t* bytes);
 
 /* Queue a request; fails with BGK_ENOMEM if it can never fit the budget. */
