@@ -8,13 +8,13 @@
 // whose two lattices live in one device arena sized by the caller's HBM
 // budget; requests are admitted in arrival order while the arena can hold
 // them.  The requests of a chunk are split by (storage type, rounding, row
-// layout) group into sub-batches of at most 256 MB of lattices, and each
-// sub-batch runs all the chunk's steps, one launch per step or per two
-// (collide_pair, by the engine's rule), before the next.  A request alone in its sub-batch runs the engine's own kernel; the
-// launch grid of a larger sub-batch is the concatenation of its requests'
-// row blocks, and a block finds its request through a per-block owner table
-// and then runs the same per-cell code as the single-request kernel.  So a
-// request's result does not depend on what it shares the GPU with
+// layout) group into sub-batches of at most 512 MB of lattices (256 MB with two
+// steps per launch: collide_pair, by the engine's rule), and each sub-batch runs
+// all the chunk's steps, one launch per step or per two, before the next.  A
+// request alone in its sub-batch runs the engine's own kernel; the launch grid
+// of a larger sub-batch is the concatenation of its requests' row blocks, and a
+// block finds its request through a per-block owner table and then runs the
+// same per-cell code as the single-request kernel.  So a request's result does not depend on what it shares the GPU with
 // (stochastic-rounding streams are keyed by cell index, request seed and
 // the request's own step count).
 //
@@ -56,17 +56,19 @@ constexpr int kServeWaves = 6;
 constexpr size_t kArenaAlign = 64 << 10;
 // A chunk runs its steps sub-batch by sub-batch: consecutive requests of a
 // storage group whose lattices add up to at most this many bytes (one larger
-// request forms its own), each sub-batch all K steps before the next: what
-// the 256 MB last-level cache holds (keep_in_cache; FP32 cavities of 98^3 and
-// 109^3 take 51 us per step together, 20 and 21 one after the other).  One
-// step per launch, too, streams faster over a small working set, whose address
-// translations stay cached from one launch to the next (16-request cavity mix,
-// FP32 part: 30.9k MLUPS with 512 MB sub-batches, 28.1k with 3 GB).  Every
-// request advances the chunk's steps in order, so results do not depend on
-// the grouping.  A request alone in its sub-batch runs the engine's own kernel
-// (no block-to-request lookup); batching in one launch pays only for requests
-// too small to fill the GPU by themselves.
-constexpr size_t kSubBatchBytes = size_t(1) << 28;
+// request forms its own), each sub-batch all K steps before the next.  Two
+// steps per launch: what the 256 MB last-level cache holds (keep_in_cache; FP32
+// cavities of 98^3 and 109^3 take 51 us per step together, 20 and 21 one after
+// the other).  One step per launch streams faster over a small working set too,
+// whose address translations stay cached from one launch to the next
+// (16-request cavity mix, FP32 part: 30.9k MLUPS with 512 MB sub-batches, 28.1k
+// with 3 GB), but with 256 MB it lacks blocks (six FP16 cavities of 32 ...
+// 150^3, 200 steps: 20.6 against 22.5 ms).  Every request advances the chunk's
+// steps in order, so results do not depend on the grouping.  A request alone
+// in its sub-batch runs the engine's own kernel (no block-to-request lookup);
+// batching in one launch pays only for requests too small to fill the GPU by
+// themselves.
+constexpr size_t sub_batch_bytes(bool pair) { return size_t(1) << (pair ? 28 : 29); }
 // Requests admitted at once: each holds one non-finite flag word.
 constexpr int kMaxFlags = 4096;
 // Shortest-first aging: chunks a request may be passed over in a row.
@@ -305,7 +307,7 @@ int prepare_group(bgks_server& s, bgks_server::Group& g, const std::vector<Insta
     const bool pair = !members.empty() && members[0]->h.pair;
     for (size_t q = 0; q < members.size(); ++q) {
         bgk_handle& h = members[q]->h;
-        if (subs.empty() || (sub_bytes > 0 && sub_bytes + members[q]->len > kSubBatchBytes)) {
+        if (subs.empty() || (sub_bytes > 0 && sub_bytes + members[q]->len > sub_batch_bytes(pair))) {
             subs.push_back({total, 0, 0, 0, (int)q, 0});
             sub_bytes = 0;
         } else {

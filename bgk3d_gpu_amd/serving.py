@@ -4,8 +4,8 @@
 (bgks_*): requests are admitted within an HBM budget (arrival order, or
 shortest remaining work first with aging) and the scheduled requests
 advance with one kernel launch per storage group, step or two and sub-batch
-of at most 256 MB; a request whose solution turns non-finite is retired at the end
-of that chunk.  `run_batched` drives it over a request stream;
+of at most 512 MB (256 MB with two steps per launch); a request whose solution
+turns non-finite is retired at the end of that chunk.  `run_batched` drives it over a request stream;
 `run_sequential` is the plain loop the reference's sweep script stands for
 (UTIL/run_sweep.sh:55-63, 128-169): one solve after the other, each with its
 own handle (allocate, rest start, `steps` time steps, diagnostics, free).

@@ -160,10 +160,10 @@ const char* bgk_last_error(void);
  *
  * Requests are admitted while the device arena reserved by bgks_create (the
  * HBM budget) can hold their two lattices; the requests scheduled for a
- * chunk advance sub-batch by sub-batch (at most 256 MB of lattices of one
- * storage, rounding and row layout), one kernel launch per sub-batch and
- * step or two steps, on one stream; requests join and leave between chunks of at
- * most chunk_steps steps, cut shorter by a chunk-time target if one is set
+ * chunk advance sub-batch by sub-batch (at most 512 MB of lattices of one
+ * storage, rounding and row layout, 256 MB with two steps per launch), one
+ * kernel launch per sub-batch and step or two steps, on one stream; requests
+ * join and leave between chunks of at most chunk_steps steps, cut shorter by a chunk-time target if one is set
  * (see enum bgks_policy).  A request whose populations turn non-finite (the
  * step kernel checks every cell) is retired as unstable at the end of that
  * chunk.  A request's populations are bit-identical to those of a handle

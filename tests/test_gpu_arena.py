@@ -1,5 +1,6 @@
-"""The server's arena: what a request holds beyond request_bytes, and the
-holes that finished ones leave, keep nobody waiting."""
+"""The server's arena and launches: what a request holds beyond request_bytes,
+and the holes that finished ones leave, keep nobody waiting; requests of one
+step per launch share launches up to 512 MB."""
 import numpy as np
 import pytest
 
@@ -87,3 +88,15 @@ def test_holes_are_gathered(gpu):
             dirs = (0, 6, 13, 18)
             for d, ref in zip(dirs, alone(r, dirs)):
                 assert np.array_equal(srv.population(q, d, r.n), ref), (r.n, d)
+
+
+def test_one_step_requests_share_launches(gpu):
+    """Two FP16 requests of 436 MB together, more than the last-level cache
+    holds: one launch a step, which fills the GPU."""
+    reqs = [S.Request(140, 200.0 + q, "f16", 10) for q in range(2)]
+    assert 1 << 28 < sum(S.request_bytes(r) for r in reqs) < 1 << 29
+    with S.Server(1 << 30, 10) as srv:
+        for r in reqs:
+            srv.submit(r)
+        assert len(srv.advance()) == 2
+        assert srv.stats()["launches"] == 10
