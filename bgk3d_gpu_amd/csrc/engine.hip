@@ -700,12 +700,12 @@ int bgk_diagno(bgk_handle* h, double out[5])
 {
     if (!h || !out) return fail(BGK_EINVAL, "bad arguments");
     ENG_HIP(hipSetDevice(h->cfg.device));
-    const int nb = diagno_blocks((long)h->cfg.m * h->cfg.n);
+    const DiagnoGrid dg = diagno_grid(h->cfg.l, (long)h->cfg.m * h->cfg.n);
     int rc = by_storage(h->cfg, [&](auto tag) {
         typedef decltype(tag) S;
-        hipLaunchKernelGGL(diagno_partial<S>, dim3(nb), dim3(kRedThreads), 0, h->stream, h->current<S>(), h->geom(),
-                           cte_one<S>(), h->scratch);
-        hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, h->stream, h->scratch, nb, h->hscratch);
+        launch_diagno(h->current<S>(), h->geom(), cte_one<S>(), dg, h->scratch, h->stream);
+        hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, h->stream, h->scratch, dg.blocks,
+                           h->hscratch);
         return 0;
     });
     if (rc) return rc;

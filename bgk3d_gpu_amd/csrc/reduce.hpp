@@ -72,9 +72,23 @@ __global__ __launch_bounds__(kRedThreads) void fold_partials(const double* __res
     }
 }
 
-// Blocks of diagno_partial: a wave per row of cells, at most kRedBlocks
-// blocks of four waves (then a wave takes several rows).
-inline int diagno_blocks(long rows) { return (int)((rows + 3) / 4 < kRedBlocks ? (rows + 3) / 4 : kRedBlocks); }
+// Threads per row of cells and blocks of diagno_partial, at most kRedBlocks
+// (then the threads of a row take several).  A wave per row:
+// rows shorter than a block's 256 threads leave none of them idle.  A block
+// per row while that takes no more blocks than CUs, or two per CU for rows
+// whose cells one wave would walk in more than 8 loads (us, a wave against a
+// block per row: FP32 130 cells, 256 rows 19.5 / 18.5, 1024 rows 19.7 / 21.6; 600
+// cells, 529 rows 22.9 / 21.8, 1024 rows 25.6 / 25.9; 2500 cells, 256 rows 38.7 /
+// 25.1; FP64 300 cells, 1024 rows 25.1 / 26.2; 2500 cells, 256 rows 44.5 / 31.7).
+struct DiagnoGrid {
+    int span, blocks;
+};
+inline DiagnoGrid diagno_grid(int l, long rows)
+{
+    const int span = l > 64 && rows <= (l > 512 ? 512 : 256) ? kRedThreads : 64;
+    const long per = kRedThreads / span, blocks = (rows + per - 1) / per;
+    return {span, (int)(blocks < kRedBlocks ? blocks : kRedBlocks)};
+}
 
 // The 19 stored values of cell s.
 template <typename S>
@@ -86,13 +100,12 @@ __device__ __forceinline__ void load_cell(const Lattice19<S>& a, long s, typenam
 
 // diagno (SRC/diagno.F90:89-131): per interior cell rho, u, v, w and
 // 0.5|u|^2 in the storage kind; partial sums {u, v, w, rho, ke} in FP64.
-// A wave takes a row (j, k) at a time, its lanes walk i: rows shorter than a
-// block's 256 threads leave none of them idle.  With varm below (one read of
-// the lattice instead of two, by all CUs) and the results of every diagnostic
-// written to host memory by its last kernel, the set printed at a check
-// (means, plane means, three lines, a probe, drag) took 410 us at 450 x 150 x
-// 150 FP32 instead of 815.
-template <typename S>
+// SPAN threads take a row (j, k) at a time and walk i (diagno_grid).  With
+// varm below (one read of the lattice instead of two, by all CUs) and the
+// results of every diagnostic written to host memory by its last kernel, the
+// set printed at a check (means, plane means, three lines, a probe, drag) took
+// 410 us at 450 x 150 x 150 FP32 instead of 815.
+template <typename S, int SPAN>
 __global__ __launch_bounds__(kRedThreads) void diagno_partial(Lattice19<S> a, Geometry g,
                                                               typename Storage<S>::compute cte1,
                                                               double* __restrict__ part)
@@ -100,10 +113,10 @@ __global__ __launch_bounds__(kRedThreads) void diagno_partial(Lattice19<S> a, Ge
     typedef typename Storage<S>::compute R;
     double v[5] = {0, 0, 0, 0, 0};
     const long rows = (long)g.m * g.n;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (long r = (long)blockIdx.x * 4 + wave; r < rows; r += (long)gridDim.x * 4) {
+    constexpr int PER = kRedThreads / SPAN;
+    for (long r = (long)blockIdx.x * PER + threadIdx.x / SPAN; r < rows; r += (long)gridDim.x * PER) {
         const int j = 1 + (int)(r % g.m), k = 1 + (int)(r / g.m);
-        for (int i = 1 + lane; i <= g.l; i += 64) {
+        for (int i = 1 + threadIdx.x % SPAN; i <= g.l; i += SPAN) {
             R x[19];
             load_cell(a, gidx(g, i, j, k), x);
             const R rho = density_ref(x, cte1);
@@ -123,6 +136,17 @@ __global__ __launch_bounds__(kRedThreads) void diagno_partial(Lattice19<S> a, Ge
 #pragma unroll
         for (int q = 0; q < 5; ++q) part[(long)blockIdx.x * 5 + q] = v[q];
     }
+}
+
+template <typename S>
+void launch_diagno(const Lattice19<S>& a, const Geometry& g, typename Storage<S>::compute cte1, const DiagnoGrid& dg,
+                   double* part, hipStream_t stream)
+{
+    if (dg.span == kRedThreads)
+        hipLaunchKernelGGL((diagno_partial<S, kRedThreads>), dim3(dg.blocks), dim3(kRedThreads), 0, stream, a, g, cte1,
+                           part);
+    else
+        hipLaunchKernelGGL((diagno_partial<S, 64>), dim3(dg.blocks), dim3(kRedThreads), 0, stream, a, g, cte1, part);
 }
 
 // Rows whose varm sums are held at a time (32 bytes each, 8 MB): longer

@@ -430,11 +430,10 @@ int diagno_gpu(real_t** a, int l, int m, int n, int nx, int ny, real_t cte1, dou
     if (!shape_ok("diagno_gpu", l, m, n, nx, ny, a) || !out) return -1;
     double *dev = nullptr, *host = nullptr;
     if (!cached_scratch((size_t)kRedBlocks * 5, 5, &dev, &host)) return -2;
-    const int nb = diagno_blocks((long)m * n);
-    hipLaunchKernelGGL(diagno_partial<real_t>, dim3(nb), dim3(kRedThreads), 0, abi_stream(), lat_from(a),
-                       geom(l, m, n, nx, ny), cte1, dev);
+    const DiagnoGrid dg = diagno_grid(l, (long)m * n);
+    launch_diagno(lat_from(a), geom(l, m, n, nx, ny), cte1, dg, dev, abi_stream());
     report_launch("diagno_partial");
-    hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, abi_stream(), dev, nb, host);
+    hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, abi_stream(), dev, dg.blocks, host);
     report_launch("fold_partials");
     if (int rc = finish()) return rc;
     diagno_means(host, l, m, n, out);
@@ -444,7 +443,8 @@ int diagno_gpu(real_t** a, int l, int m, int n, int nx, int ny, real_t cte1, dou
 int diagno_gpu_noalloc(real_t** a, int l, int m, int n, int nx, int ny, real_t cte1, double* out)
 {
     if (!shape_ok("diagno_gpu_noalloc", l, m, n, nx, ny, a) || !out) return -1;
-    const int nb = diagno_blocks((long)m * n);
+    const DiagnoGrid dg = diagno_grid(l, (long)m * n);
+    const int nb = dg.blocks;
     // the partials of nb blocks after the 5 totals
     if ((size_t)(nb + 1) * 5 > kNoAllocDoubles) {
         std::fprintf(stderr, "bgk3d_gpu: diagno_gpu_noalloc: %d partials exceed the static scratch of %zu doubles\n",
@@ -454,8 +454,7 @@ int diagno_gpu_noalloc(real_t** a, int l, int m, int n, int nx, int ny, real_t c
     double* dev = noalloc_scratch_ptr();
     if (!dev) return -2;
     // every partial and total is written before it is read: nothing to clear
-    hipLaunchKernelGGL(diagno_partial<real_t>, dim3(nb), dim3(kRedThreads), 0, abi_stream(), lat_from(a),
-                       geom(l, m, n, nx, ny), cte1, dev + 5);
+    launch_diagno(lat_from(a), geom(l, m, n, nx, ny), cte1, dg, dev + 5, abi_stream());
     report_launch("diagno_partial");
     hipLaunchKernelGGL(fold_partials<5>, dim3(1), dim3(kRedThreads), 0, abi_stream(), dev + 5, nb, dev);
     report_launch("fold_partials");
