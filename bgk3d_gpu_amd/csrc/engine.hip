@@ -246,6 +246,24 @@ bool collide_fills_faces(const bgk_handle& h)
     return h.cfg.les ? kFillsInflowFaces<S, 4> : kFillsInflowFaces<S, 0>;
 }
 
+// Rows for a call of `steps` steps of a handle that can have either.  Two steps
+// per launch need padded rows and save about 0.7 of a step each time; a step
+// alone takes 3 ... 23 % longer on them (us per step in calls of one step,
+// compact against padded rows: FP32 130^3 60.4 / 68.5, 97 x 97 x 140 36.7 / 45.3,
+// 200^3 204 / 223, 420 x 199 x 180 372 / 414; MIXED2 200^3 204 / 230; FP64 150^3 177 /
+// 184).  The move takes about 1.5 steps, so it comes when the calls since the
+// last one would have saved that much: before a long call at once, and back
+// after some 15 calls of one step.
+int choose_rows(bgk_handle& h, int steps)
+{
+    if (!h.flex) return 0;
+    const double saved = 0.7 * (steps / 2) - 0.1 * (steps % 2);
+    h.owed = std::max(0.0, h.owed + (h.compact ? saved : -saved));
+    if (h.owed < 1.5) return 0;
+    h.owed = 0;
+    return relayout(h, !h.compact);
+}
+
 // queue the boundary work and the fused collide of one step, or of two in
 // one pass where that is faster and two are left, then swap; returns the
 // steps taken.  `first`: the first launch of a stepping call, after which
@@ -254,7 +272,7 @@ bool collide_fills_faces(const bgk_handle& h)
 template <typename S>
 int one_launch(bgk_handle& h, int left, hipEvent_t pre, hipEvent_t post, bool first)
 {
-    const bool pair = h.pair && left >= 2;
+    const bool pair = h.pair && !h.compact && left >= 2;
     if (h.cfg.boundary == BGK_BC_INFLOW && (first || pair || !collide_fills_faces<S>(h))) {
         hipLaunchKernelGGL(outflow_halo<S>, dim3(ceil_div((long)h.cfg.m * h.cfg.n, 256)), dim3(256), 0, h.stream,
                            h.current<S>(), h.geom(), h.compact, (typename Storage<S>::compute)h.u_inflow);
@@ -424,9 +442,10 @@ int handle_setup(bgk_handle& h, const bgk_config& c, bool roomy)
     // Rows padded to whole lines, or compact rows where those measured
     // faster (prefer_compact: enough of a row's last line unused, or, with
     // 32/64-bit storage, a lattice of 2^24 cells or more).  Lattices that
-    // take two steps per launch keep padded rows: the tiles of collide_pair
+    // take two steps per launch have padded rows: the tiles of collide_pair
     // start and end on lines (413 against 346 us per FP32 step at 256^3 over
-    // compact rows).
+    // compact rows).  They turn to compact rows where the caller takes one
+    // step at a time (choose_rows).
     const double waste = (double)(round_up(c.l, h.A) - c.l) / (double)c.l;
     const bool compact = c.layout == 2 || (c.layout == 0 && prefer_compact(c, waste));
     h.pair = (roomy || !compact) && prefer_pair(c, round_up(c.l + 2, h.A) * h.ny, h.pgrid);
@@ -646,6 +665,7 @@ int bgk_step(bgk_handle* h, int nsteps)
 {
     if (!h || nsteps < 0) return fail(BGK_EINVAL, "bad arguments");
     ENG_HIP(hipSetDevice(h->cfg.device));
+    if (int rc = choose_rows(*h, nsteps)) return rc;
     return by_storage(h->cfg, [&](auto tag) {
         for (int s = 0; s < nsteps;) s += one_launch<decltype(tag)>(*h, nsteps - s, nullptr, nullptr, s == 0);
         hipError_t e = hipGetLastError();
@@ -673,6 +693,7 @@ int bgk_time_steps(bgk_handle* h, int nsteps, double* total_ms, double* collide_
     ENG_HIP(hipStreamSynchronize(h->stream));
     hipEvent_t e0 = h->events[0], e1 = h->events[1];
     ENG_HIP(hipEventRecord(e0, h->stream));
+    if (int rc = choose_rows(*h, nsteps)) return rc;
     int launches = 0;
     int rc = by_storage(h->cfg, [&](auto tag) {
         for (int s = 0; s < nsteps; ++launches)

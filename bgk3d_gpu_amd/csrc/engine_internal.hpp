@@ -42,6 +42,7 @@ struct bgk_handle {
     // `flex`: one step at a time would run on compact rows; lstride holds a
     // lattice of either rows (relayout)
     bool pair = false, flex = false;
+    double owed = 0;  // steps that the other rows would have saved (choose_rows)
     bgk::PairGrid pgrid{};
     void* mem[2] = {nullptr, nullptr};
     size_t bytes = 0;

@@ -65,14 +65,15 @@ typedef struct bgk_config {
                              reference's expression order (the plain F16 form uses a leaner
                              FP32 arithmetic); 2 MIXED2: storage BGK_F32, collision in FP64 */
     int layout;           /* 0 choose, 1 rows padded to 128-byte lines, 2 compact rows of l + 2
-                             cells.  The default takes padded rows
-                             where two steps per launch run faster (FP32 and FP64 storage, from
-                             about 32^3 up), else compact rows
-                             where they measured faster: when padding would leave more than 3 %
-                             of a row unused in its last line (9 % with 16-bit storage; a line
-                             holds 32 values in FP32, 16 in FP64, 64 in 16-bit storage), and
-                             with FP32/FP64 storage for lattices of 2^24 cells or more, or where
-                             the padded lattice cannot be allocated */
+                             cells.  The default takes padded rows where two steps per launch
+                             are estimated to run faster (FP32 and FP64 storage), else compact
+                             rows where they measured faster: when padding would leave more than
+                             3 % of a row unused in its last line (9 % with 16-bit storage; a
+                             line holds 32 values in FP32, 16 in FP64, 64 in 16-bit storage), and
+                             with FP32/FP64 storage for lattices of 2^24 cells or more.  Where
+                             both hold, the handle turns to compact rows after some 15 calls of
+                             one step, and back before a call of several; where the padded
+                             lattice cannot be allocated it has compact rows throughout */
 } bgk_config;
 
 typedef struct bgk_handle bgk_handle;
@@ -145,7 +146,7 @@ int bgk_get_population(bgk_handle* h, int d, double* out);
 /* Overwrite interior values of population d (rounded to the storage type). */
 int bgk_set_population(bgk_handle* h, int d, const double* in);
 
-/* Sizes: [0] nx, [1] ny, [2] nz, [3] bytes of device memory held,
+/* Sizes: [0] nx (of the present rows), [1] ny, [2] nz, [3] bytes of device memory held,
  * [4] storage bytes per population value, [5] steps taken. */
 int bgk_info(bgk_handle* h, long long out[6]);
 
