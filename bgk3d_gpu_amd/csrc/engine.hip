@@ -474,6 +474,23 @@ int handle_setup(bgk_handle& h, const bgk_config& c, bool roomy)
     return 0;
 }
 
+// Set up `h` where `free_bytes` of the device are free.  The padded rows of two
+// steps per launch, up to 40 % more memory than compact rows, are taken only
+// where the room they leave is at least eight times what they take beyond
+// those, and 64 MB: what a program allocates next (the 8 bytes a cell of
+// bgk_get_population; another handle) finds at least 8/9 of the room that it
+// had beside compact rows.
+static int setup_within(bgk_handle& h, const bgk_config& c, size_t free_bytes)
+{
+    if (int rc = handle_setup(h, c)) return rc;
+    if (!h.flex) return 0;
+    bgk_handle small;
+    if (int rc = handle_setup(small, c, false)) return rc;
+    const size_t padded = lattice_bytes(h), extra = padded - lattice_bytes(small);
+    if (extra && free_bytes < padded + 8 * extra + (size_t(64) << 20)) return handle_setup(h, c, false);
+    return 0;
+}
+
 int join_rest(bgk_handle& h)
 {
     if (h.rest == h.cur) return 0;
@@ -538,6 +555,19 @@ void bgk_config_default(bgk_config* c, int l, int m, int n)
 
 const char* bgk_last_error(void) { return last_error(); }
 
+int bgk_plan(const bgk_config* cfg, size_t free_bytes, long long out[5])
+{
+    if (!cfg || !out) return fail(BGK_EINVAL, "null argument");
+    bgk_handle h;
+    if (int rc = setup_within(h, *cfg, free_bytes)) return rc;
+    out[0] = h.pair ? 2 : 1;
+    out[1] = h.compact;
+    out[2] = (long long)lattice_bytes(h);
+    out[3] = h.pair ? h.pgrid.th : 0;
+    out[4] = h.pair ? h.pgrid.zc : 0;
+    return 0;
+}
+
 int bgk_create(const bgk_config* cfg, bgk_handle** out)
 {
     if (!cfg || !out) return fail(BGK_EINVAL, "null argument");
@@ -557,6 +587,8 @@ int bgk_create(const bgk_config* cfg, bgk_handle** out)
         delete h;
         return fail(BGK_EHIP, "hipSetDevice(%d) failed", c.device);
     }
+    size_t free_bytes = 0, total = 0;
+    if (h->flex && hipMemGetInfo(&free_bytes, &total) == hipSuccess) (void)setup_within(*h, c, free_bytes);
 
     int rc = 0;
     auto cleanup = [&](int code) {

@@ -36,6 +36,7 @@ def lib() -> ctypes.CDLL:
         vp, ci, dp = ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_double)
         L.bgk_config_default.argtypes = [ctypes.POINTER(BGKConfig), ci, ci, ci]
         L.bgk_config_default.restype = None
+        L.bgk_plan.argtypes = [ctypes.POINTER(BGKConfig), ctypes.c_size_t, ctypes.POINTER(ctypes.c_longlong)]
         L.bgk_create.argtypes = [ctypes.POINTER(BGKConfig), ctypes.POINTER(vp)]
         L.bgk_destroy.argtypes = [vp]
         L.bgk_step.argtypes = [vp, ci]
@@ -94,6 +95,14 @@ def make_config(case: Case, storage: str = "f32", rounding: int = 0, obstacle: i
     c.mixed = mixed
     c.layout = layout
     return c
+
+
+def plan(case: Case, storage: str = "f32", free_bytes: int = 1 << 60, **kw) -> dict:
+    """What Engine(case, storage, **kw) would choose with free_bytes of the
+    device free (no GPU needed)."""
+    out = (ctypes.c_longlong * 5)()
+    _check(lib().bgk_plan(ctypes.byref(make_config(case, storage, **kw)), free_bytes, out), "bgk_plan")
+    return dict(steps_per_launch=out[0], compact=bool(out[1]), bytes=out[2], tile_rows=out[3], tile_planes=out[4])
 
 
 class Engine:

@@ -81,6 +81,15 @@ typedef struct bgk_handle bgk_handle;
 /* Fill `cfg` with the reference's defaults for a driven cavity of l x m x n. */
 void bgk_config_default(bgk_config* cfg, int l, int m, int n);
 
+/* What bgk_create would choose with free_bytes of the device free (no GPU
+ * needed): [0] steps per launch where two are left, [1] compact rows at first,
+ * [2] device bytes of the lattices, [3] rows and [4] planes of a two-step
+ * launch's tiles (0 with one step per launch).  With layout 0, two
+ * steps per launch on rows that take more memory than compact ones are chosen
+ * only if eight times the difference, and 64 MB, stay free (layout 2 for as
+ * many handles as possible on one GPU). */
+int bgk_plan(const bgk_config* cfg, size_t free_bytes, long long out[5]);
+
 int bgk_create(const bgk_config* cfg, bgk_handle** out);
 int bgk_destroy(bgk_handle* h);
 
