@@ -170,16 +170,12 @@ def bench_engine(case, storage, steps, warmup, want_ke=False, rounding=None, **k
         eng.sync()
         total_ms, kern_ms = eng.time_steps(steps)
         diag = eng.diagno()
-        info = eng.info()
+        info = {**eng.info(), **eng.launch_info()}
+        if steps < 2:
+            info["steps_per_launch"] = 1
     if want_ke:
         info["ke0"] = ke0
     return total_ms, kern_ms, diag, info
-
-
-def steps_per_launch(case, info):
-    """2 where the engine takes two steps per launch (collide_pair): FP32 and
-    FP64 storage on padded rows (it chooses compact rows for one step)."""
-    return 2 if info["esize"] >= 4 and info["nx"] != case.l + 2 else 1
 
 
 def bench_sphere(steps):
@@ -194,7 +190,7 @@ def bench_sphere(steps):
     case = Case("inflow", l, m, n, svisc=U * 2 * R / 300.0, u0=U, obstacle=True)
     t, k, d, info = bench_engine(case, "f32", steps, 3, obstacle=2, centre=(l // 4, m // 2, n // 2), radius=R,
                                  u_inflow=U)
-    per = steps_per_launch(case, info)
+    per = info["steps_per_launch"]
     out = {"sphere_engine": {"mlups": round(case.cells * steps / (t * 1e-3) / 1e6, 1),
                              "collide_us": round(k * 1e3, 1), "device_bytes": info["bytes"],
                              "steps_per_launch": per,
@@ -326,7 +322,7 @@ def main():
     ms_per_step = total_ms / args.steps
     mlups = case.cells * args.steps / (total_ms * 1e-3) / 1e6
     alg_bytes = 38 * s_bytes * case.cells
-    per_launch = steps_per_launch(case, info)
+    per_launch = info["steps_per_launch"]
     achieved = alg_bytes / (per_launch * kern_avg_ms * 1e-3) / 1e9
     log(f"MLUPS {mlups:.0f}; collide avg {kern_avg_ms * 1e3:.1f} us per step, {per_launch} per launch -> {achieved:.0f} GB/s")
     forms = {}
@@ -343,7 +339,7 @@ def main():
             if st == storage and not mixed:
                 continue
             t, k, d, finfo = bench_engine(case, st, fsteps, 5, rounding=rnd, mixed=mixed)
-            per = steps_per_launch(case, finfo)
+            per = finfo["steps_per_launch"]
             forms[name] = {"mlups": round(case.cells * fsteps / (t * 1e-3) / 1e6, 1),
                            "collide_us": round(k * 1e3, 2), "steps_per_launch": per,
                            "alg_GBs": round(38 * sb * case.cells / (per * k * 1e-3) / 1e9, 1)}
@@ -377,7 +373,7 @@ def main():
         log("cpu baseline ...")
         cpu = cpu_baseline(case, args.cpu_steps)
         log(f"cpu baseline {cpu['value']:.2f} MLUPS ({cpu['kind']}, {cpu['cores']} cores)")
-    compact = info["nx"] == n + 2  # the engine chose compact rows
+    compact = info["compact"]
     kernel = "collide_pair" if per_launch == 2 else ("collide_compact" if compact else "collide_fused")
     traffic = load_traffic(workload, kernel)
     out = {

@@ -1087,4 +1087,14 @@ int bgk_info(bgk_handle* h, long long out[6])
     return 0;
 }
 
+int bgk_launch_info(bgk_handle* h, long long out[4])
+{
+    if (!h || !out) return fail(BGK_EINVAL, "bad arguments");
+    out[0] = h->pair ? 2 : 1;
+    out[1] = h->compact;
+    out[2] = h->pair ? h->pgrid.th : 0;
+    out[3] = h->pair ? h->pgrid.zc : 0;
+    return 0;
+}
+
 }  // extern "C"

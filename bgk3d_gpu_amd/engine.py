@@ -55,6 +55,7 @@ def lib() -> ctypes.CDLL:
         L.bgk_write_vtk.argtypes = [vp, ci, ci, ctypes.c_char_p]
         L.bgk_set_population.argtypes = [vp, ci, vp]
         L.bgk_info.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
+        L.bgk_launch_info.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
         L.bgk_last_error.restype = ctypes.c_char_p
         L._bgk_typed = True
     return L
@@ -197,6 +198,12 @@ class Engine:
         out = (ctypes.c_longlong * 6)()
         _check(self.L.bgk_info(self.h, out), "bgk_info")
         return dict(nx=out[0], ny=out[1], nz=out[2], bytes=out[3], esize=out[4], steps=out[5])
+
+    def launch_info(self) -> dict:
+        """Steps per launch of a call of several steps, present rows, tiles."""
+        out = (ctypes.c_longlong * 4)()
+        _check(self.L.bgk_launch_info(self.h, out), "bgk_launch_info")
+        return dict(steps_per_launch=out[0], compact=bool(out[1]), tile_rows=out[2], tile_planes=out[3])
 
     def close(self):
         if self.h:

@@ -4,7 +4,8 @@ Periodic Taylor-Green in FP32 (handle API) at sizes from 0.7 GB to 22 GB of
 device memory: the same kernel and row length, only the number of rows and
 planes grows.  Prints one JSON line per size: bytes held, mean step and
 collide-kernel durations (hipEvents), MLUPS and the kernel's algorithmic
-bandwidth (38 x 4 bytes per cell).
+bandwidth (38 x 4 bytes per cell, once for the two steps of a collide_pair
+launch).
 
     python -m bgk3d_gpu_amd.studies.footprint > footprint.json
 """
@@ -29,10 +30,12 @@ def main(argv=None):
             info = eng.info()
             eng.time_steps(10)
             ms, kern_ms = eng.time_steps(args.steps)
+            per = eng.launch_info()["steps_per_launch"] if args.steps > 1 else 1
         cells = l * m * n
         print(json.dumps({"grid": [l, m, n], "device_bytes": info["bytes"], "step_us": ms / args.steps * 1e3,
-                          "collide_us": kern_ms * 1e3, "mlups": cells * args.steps / (ms * 1e-3) / 1e6,
-                          "alg_GBs": 38 * 4 * cells / (kern_ms * 1e-3) / 1e9}), flush=True)
+                          "collide_us": kern_ms * 1e3, "steps_per_launch": per,
+                          "mlups": cells * args.steps / (ms * 1e-3) / 1e6,
+                          "alg_GBs": 38 * 4 * cells / (per * kern_ms * 1e-3) / 1e9}), flush=True)
 
 
 if __name__ == "__main__":

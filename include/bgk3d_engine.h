@@ -159,6 +159,12 @@ int bgk_set_population(bgk_handle* h, int d, const double* in);
  * [4] storage bytes per population value, [5] steps taken. */
 int bgk_info(bgk_handle* h, long long out[6]);
 
+/* How a call of several steps is launched: [0] steps per launch (1 or 2; an
+ * odd step left takes a launch of its own), [1] whether the rows are compact at
+ * present, [2] rows and [3] planes of a two-step launch's tiles (0 with one
+ * step per launch). */
+int bgk_launch_info(bgk_handle* h, long long out[4]);
+
 /* Text of the last error on this thread. */
 const char* bgk_last_error(void);
 
