@@ -256,7 +256,7 @@ bool collide_fills_faces(const bgk_handle& h)
 // after some 15 calls of one step.
 int choose_rows(bgk_handle& h, int steps)
 {
-    if (!h.flex) return 0;
+    if (!h.flex || h.launch) return 0;
     const double saved = 0.7 * (steps / 2) - 0.1 * (steps % 2);
     h.owed = std::max(0.0, h.owed + (h.compact ? saved : -saved));
     if (h.owed < 1.5) return 0;
@@ -1084,6 +1084,34 @@ int bgk_info(bgk_handle* h, long long out[6])
     out[3] = (long long)h->bytes;
     out[4] = (long long)h->esize;
     out[5] = h->steps;
+    return 0;
+}
+
+int bgk_set_launch(bgk_handle* h, int steps, int rows, int planes)
+{
+    if (!h || steps < 0 || steps > 2 || rows < 0 || planes < 0) return fail(BGK_EINVAL, "bad arguments");
+    const bgk_config& c = h->cfg;
+    const bool padded = h->flex || !h->compact;
+    const long plane = round_up(c.l + 2, h->A) * h->ny;
+    PairGrid g{};
+    const bool rule = padded && prefer_pair(c, plane, g);
+    if (steps == 2) {
+        if (!padded || !can_pair(c, plane))
+            return fail(BGK_EINVAL, "two steps per launch need FP32 or FP64 storage on padded rows (layout 1)");
+        if (rows > pair_rows_max(c) || planes > c.n)
+            return fail(BGK_EINVAL, "tiles of %d rows, %d planes: at most %d and %d", rows, planes, pair_rows_max(c),
+                        c.n);
+        if (rows || planes) g = pair_grid_of(c.l, c.m, c.n, rows ? rows : g.th, planes ? planes : g.zc);
+        if (g.total <= 0) return fail(BGK_EINVAL, "more than 2^30 tiles");
+    } else if (rows || planes) {
+        return fail(BGK_EINVAL, "tiles are those of two steps per launch");
+    }
+    ENG_HIP(hipSetDevice(c.device));
+    if (steps && h->flex)
+        if (int rc = relayout(*h, steps == 1)) return rc;
+    h->launch = steps;
+    h->pair = steps ? steps == 2 : rule;
+    h->pgrid = g;
     return 0;
 }
 

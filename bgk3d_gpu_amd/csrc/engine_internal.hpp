@@ -42,6 +42,7 @@ struct bgk_handle {
     // `flex`: one step at a time would run on compact rows; lstride holds a
     // lattice of either rows (relayout)
     bool pair = false, flex = false;
+    int launch = 0;   // steps per launch asked for (bgk_set_launch), 0: the rule's
     double owed = 0;  // steps that the other rows would have saved (choose_rows)
     bgk::PairGrid pgrid{};
     void* mem[2] = {nullptr, nullptr};
@@ -154,6 +155,23 @@ int by_storage(const bgk_config& c, F&& f)
 // The collision runs in FP64 (DOUBLE_P storage, or the MIXED2 form).
 inline bool compute_double(const bgk_config& c) { return c.storage == BGK_F64 || c.mixed == 2; }
 
+// Whether two steps per launch can be taken at all, on padded rows with
+// `plane` values a population plane.
+inline bool can_pair(const bgk_config& c, long plane)
+{
+    const size_t es = storage_bytes(c.storage);
+    if (es < 4 || c.layout == 2) return false;
+    // a lane's 32-bit byte offset spans up to four z levels (pair_tile)
+    return 80.0 * (double)es * (double)plane < 4.0e9;
+}
+
+// Most rows of a tile.
+inline int pair_rows_max(const bgk_config& c)
+{
+    return c.storage == BGK_F64 ? PairShape<double>::TY
+                                : (compute_double(c) ? PairShape<mix32_t>::TY : PairShape<float>::TY);
+}
+
 // Tiles of the two-step kernel for this configuration, if two steps per
 // launch are faster than two launches of one.  Estimates in us from measured
 // launches: a single step takes 1.5 + its bytes at 6.2 TB/s, at least 4.6; a
@@ -167,14 +185,11 @@ inline bool compute_double(const bgk_config& c) { return c.storage == BGK_F64 ||
 // 512 x 128^2 108 / 118 with one cell per lane, 109 / 131 with two).
 inline bool prefer_pair(const bgk_config& c, long plane, PairGrid& g)
 {
+    if (!can_pair(c, plane)) return false;
     const size_t es = storage_bytes(c.storage);
     const bool wide = compute_double(c);
-    if (es < 4 || c.layout == 2) return false;
-    // a lane's 32-bit byte offset spans up to four z levels (pair_tile)
-    if (80.0 * (double)es * (double)plane >= 4.0e9) return false;
     double cost;
-    const int rows = es == 8 ? PairShape<double>::TY : (wide ? PairShape<mix32_t>::TY : PairShape<float>::TY);
-    g = pair_grid(c.l, c.m, c.n, rows, cost);
+    g = pair_grid(c.l, c.m, c.n, pair_rows_max(c), cost);
     const double cells = (double)c.l * c.m * c.n;
     const double two = 2 * std::max(4.6, 1.5 + 38.0 * (double)es * cells / 6.2e6);
     const double us = es == 8 ? (c.les ? 1.10 : 0.70) : (wide ? (c.les ? 0.53 : 0.46) : (c.les ? 0.44 : 0.42));

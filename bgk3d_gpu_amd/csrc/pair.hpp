@@ -598,6 +598,23 @@ inline PairGrid pair_grid(int l, int m, int n, int rows, double& cost, double cu
     return g;
 }
 
+// Tiles of `rows` rows (at most the kernel's TY) and `planes` planes.
+inline PairGrid pair_grid_of(int l, int m, int n, int rows, int planes)
+{
+    PairGrid g{};
+    const int left = l % kTileX;
+    const bool tail = left > 0 && left <= kTileX / 2;
+    g.tx = l / kTileX + (left > kTileX / 2 ? 1 : 0);
+    g.th = rows;
+    g.ty = ceil_div(m, rows);
+    g.ty2 = tail ? ceil_div(m, 2 * rows) : 0;
+    g.zc = planes;
+    g.cz = ceil_div(n, planes);
+    const double blocks = ((double)g.tx * g.ty + g.ty2) * g.cz;
+    g.total = blocks < 1u << 30 ? (int)blocks : 0;
+    return g;
+}
+
 inline int pair_blocks(int tiles) { return ceil_div(tiles, 8) * 8; }
 
 template <typename S, int BX, int BY, int BZ, bool OB, int FM, bool NT = true>

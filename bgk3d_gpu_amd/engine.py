@@ -55,6 +55,7 @@ def lib() -> ctypes.CDLL:
         L.bgk_write_vtk.argtypes = [vp, ci, ci, ctypes.c_char_p]
         L.bgk_set_population.argtypes = [vp, ci, vp]
         L.bgk_info.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
+        L.bgk_set_launch.argtypes = [vp, ci, ci, ci]
         L.bgk_launch_info.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
         L.bgk_last_error.restype = ctypes.c_char_p
         L._bgk_typed = True
@@ -198,6 +199,11 @@ class Engine:
         out = (ctypes.c_longlong * 6)()
         _check(self.L.bgk_info(self.h, out), "bgk_info")
         return dict(nx=out[0], ny=out[1], nz=out[2], bytes=out[3], esize=out[4], steps=out[5])
+
+    def set_launch(self, steps: int, rows: int = 0, planes: int = 0):
+        """Steps per launch (1, 2, or 0 for the library's choice) and, with 2,
+        the rows and planes of a tile (0 for the library's choice)."""
+        _check(self.L.bgk_set_launch(self.h, steps, rows, planes), "bgk_set_launch")
 
     def launch_info(self) -> dict:
         """Steps per launch of a call of several steps, present rows, tiles."""

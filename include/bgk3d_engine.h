@@ -165,6 +165,12 @@ int bgk_info(bgk_handle* h, long long out[6]);
  * step per launch). */
 int bgk_launch_info(bgk_handle* h, long long out[4]);
 
+/* Launch calls of several steps with `steps` steps per launch: 1, 2 (FP32 and
+ * FP64 storage on padded rows; else BGK_EINVAL), 0 the library's choice again.
+ * rows, planes: of a two-step launch's tiles, at most 13 rows (8 in FP64, 9
+ * in MIXED2); 0 the library's choice.  Results do not depend on any of them. */
+int bgk_set_launch(bgk_handle* h, int steps, int rows, int planes);
+
 /* Text of the last error on this thread. */
 const char* bgk_last_error(void);
 
