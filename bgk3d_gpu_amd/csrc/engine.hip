@@ -356,7 +356,7 @@ int download_fields(bgk_handle& h, double* const (&outs)[4])
     std::atomic<int> next{0}, bad{0};
     auto work = [&](int w) {
         hipEvent_t done = nullptr;
-        (void)hipGetLastError();  // what an earlier call of this thread left is not this launch's
+        forget_error();
         bool ok = hipSetDevice(h.cfg.device) == hipSuccess &&
                   hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess;
         C *d = dev + slot * w, *p = host + slot * w;
@@ -587,6 +587,7 @@ int bgk_create(const bgk_config* cfg, bgk_handle** out)
         delete h;
         return fail(BGK_EHIP, "hipSetDevice(%d) failed", c.device);
     }
+    forget_error();
     size_t free_bytes = 0, total = 0;
     if (h->flex && hipMemGetInfo(&free_bytes, &total) == hipSuccess) (void)setup_within(*h, c, free_bytes);
 
@@ -600,7 +601,7 @@ int bgk_create(const bgk_config* cfg, bgk_handle** out)
     void* region = nullptr;
     hipError_t got = hipMalloc(&region, lattice_bytes(*h));
     if (got != hipSuccess && h->pair) {  // padded rows do not fit: compact ones may
-        (void)hipGetLastError();
+        forget_error();
         handle_setup(*h, c, false);
         got = hipMalloc(&region, lattice_bytes(*h));
     }
@@ -697,6 +698,7 @@ int bgk_step(bgk_handle* h, int nsteps)
 {
     if (!h || nsteps < 0) return fail(BGK_EINVAL, "bad arguments");
     ENG_HIP(hipSetDevice(h->cfg.device));
+    forget_error();
     if (int rc = choose_rows(*h, nsteps)) return rc;
     return by_storage(h->cfg, [&](auto tag) {
         for (int s = 0; s < nsteps;) s += one_launch<decltype(tag)>(*h, nsteps - s, nullptr, nullptr, s == 0);
@@ -723,6 +725,7 @@ int bgk_time_steps(bgk_handle* h, int nsteps, double* total_ms, double* collide_
         h->events.push_back(e);
     }
     ENG_HIP(hipStreamSynchronize(h->stream));
+    forget_error();
     hipEvent_t e0 = h->events[0], e1 = h->events[1];
     ENG_HIP(hipEventRecord(e0, h->stream));
     if (int rc = choose_rows(*h, nsteps)) return rc;
@@ -1107,6 +1110,7 @@ int bgk_set_launch(bgk_handle* h, int steps, int rows, int planes)
         return fail(BGK_EINVAL, "tiles are those of two steps per launch");
     }
     ENG_HIP(hipSetDevice(c.device));
+    forget_error();
     if (steps && h->flex)
         if (int rc = relayout(*h, steps == 1)) return rc;
     h->launch = steps;

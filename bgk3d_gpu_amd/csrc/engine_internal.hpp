@@ -109,6 +109,10 @@ int fail(int code, const char* fmt, ...);
         if (_e != hipSuccess) return ::bgk::eng::fail(BGK_EHIP, "%s: %s", #call, hipGetErrorString(_e)); \
     } while (0)
 
+// Drop the HIP error that an earlier call of this thread left (a handle that
+// did not fit, another library's query): the launch checks read the last one.
+inline void forget_error() { (void)hipGetLastError(); }
+
 inline size_t storage_bytes(int kind)
 {
     switch (kind) {

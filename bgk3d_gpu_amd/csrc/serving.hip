@@ -757,6 +757,7 @@ int bgks_advance(bgks_server* s, long long* done_ids, int max_done, int* n_done)
     if (!s) return fail(BGK_EINVAL, "null server");
     if (n_done) *n_done = 0;
     ENG_HIP(hipSetDevice(s->device));
+    forget_error();
     if (int rc = admit(*s)) return rc;
 
     std::vector<Instance*> active;

@@ -95,3 +95,30 @@ def test_varm_in_several_passes(gpu, size, prec):
         mag = np.abs(per[q]).sum(axis=(1, 2)) * rvol
         assert np.all(np.abs(got - per[q].sum(axis=(1, 2)) * rvol) <= 1e-12 * mag), q
     np.testing.assert_allclose(den, per["rho"].sum(axis=(0, 2)) * rvol, rtol=1e-12)
+
+
+def test_calls_after_a_refused_handle(gpu):
+    """Stepping, creating, serving and moving rows after one."""
+    from bgk3d_gpu_amd import serving as S
+
+    case = Case("periodic", 70, 30, 24, svisc=0.03, u0=0.1, init=1)
+
+    def refuse():
+        with pytest.raises(rt.BGKError):
+            Engine(Case("ldc", 4000, 4000, 4000, svisc=0.05, u0=0.1), "f64")
+
+    with Engine(case, "f32") as eng:
+        refuse()
+        eng.step(2)
+        refuse()
+        eng.time_steps(4)
+        refuse()
+        eng.set_launch(1)
+        refuse()
+        with Engine(case, "f32") as other:
+            other.step(6)
+            assert np.array_equal(eng.populations(), other.populations())
+        with S.Server(1 << 28, 10) as srv:
+            rid = srv.submit(S.Request(30, 200.0, "f32", 10))
+            refuse()
+            assert srv.advance() == [rid]
