@@ -177,16 +177,26 @@ inline int pair_rows_max(const bgk_config& c)
 }
 
 // Tiles of the two-step kernel for this configuration, if two steps per
-// launch are faster than two launches of one.  Estimates in us from measured
-// launches: a single step takes 1.5 + its bytes at 6.2 TB/s, at least 4.6; a
-// pair 2.5 + its cost (pair_grid) times 0.42 in FP32 (0.37 ... 0.43 over
-// cavities, Taylor-Green, channel and the sphere, 64^3 ... 512^3), 0.46
-// in MIXED2 and 0.70 in FP64 (0.63 ... 0.72); with LES 0.44, 0.53 and 1.10
-// (more values live than registers).  Measured per step, one step a launch
-// against two: FP32 256^3 410 / 268, 192^3 175 / 112, 64^3 9.7 / 6.3, FP64 192^3
-// 359 / 207; LES 128^3 MIXED2 60.7 / 47.5, FP64 109 / 95.  16-bit storage stays
-// with one: its kernels are bound by issue as much as by HBM (FP16 channel at
-// 512 x 128^2 108 / 118 with one cell per lane, 109 / 131 with two).
+// launch are estimated to be faster than two launches of one.  Estimates in
+// us: a single step takes 1.5 + its bytes at 6.2 TB/s, at least 4.6; a pair 2.5 +
+// its cost (pair_grid) times 0.42 in FP32, 0.46 in MIXED2 and 0.70 in FP64; with
+// LES 0.44, 0.53 and 1.10 (more values live than registers).  Both are fitted
+// to lattices that stream: above 256 MB the pair's factors measured 0.38 ...
+// 0.42, 0.39 ... 0.45, 0.55 ... 0.74 (LES 0.40 ... 0.47, 0.46 ... 0.54, 0.92 ... 1.15),
+// a single step 1.00 ... 1.25 of its estimate.  From 80 to 256 MB, where the
+// pair's stores stay in the cache (keep_in_cache), they are 0.28 ... 0.40, 0.34
+// ... 0.44, 0.51 ... 0.63 (0.33 ... 0.44, 0.43 ... 0.54, 0.72 ... 0.95) and 1.05 ... 1.35, and
+// below that they scatter: there the rule refuses lattices that two steps per
+// launch would serve better.  Over 504 lattices (24^3 ... 200^3 and flat or long
+// boxes, six forms, with bgk_set_launch) it took two only where that is faster,
+// and refused it 201 times where it is by more than 3 %.  Measured per step, one
+// step a launch against two: taken FP32 256^3 410 / 268, 150^3 88 / 64, 64^3 9.6 /
+// 6.1, FP64 192^3 359 / 207, 80^3 29.4 / 18.3; LES 128^3 MIXED2 60.7 / 47.5, FP64
+// 109 / 95; refused FP32 40^3 5.8 / 4.5, 80^3 17.6 / 11.8, 97^3 28.1 / 17.5, 100^3 29.6
+// / 20.2, FP64 56^3 12.9 / 8.6, MIXED2 100^3 28.8 / 25.9, 140^3 LES MIXED2 77 / 71.
+// 16-bit storage stays with one: its kernels are bound by issue as much as by
+// HBM (FP16 channel at 512 x 128^2 108 / 118 with one cell per lane, 109 / 131
+// with two).
 inline bool prefer_pair(const bgk_config& c, long plane, PairGrid& g)
 {
     if (!can_pair(c, plane)) return false;
@@ -235,10 +245,11 @@ inline size_t lattice_bytes(const bgk_handle& h) { return (size_t)h.lstride * 2 
 // Whether the lattices a launch works on, `bytes` together, are stored with
 // plain instead of streaming stores: the next step then finds them in the
 // 256 MB last-level cache.  Above that streaming is faster, and below 80 MB
-// too (FP32, two steps per launch, us per step, streaming against plain: 48^3
-// 5.7 / 6.2, 64^3 6.4 / 6.7, 80^3 15.0 / 12.0, 100^3 25.0 / 20.2, 112^3 30.4 / 23.4,
-// 128^3 (411 MB) 36.0 / 37.9; FP64 64^3 (106 MB) 10.7 / 10.8, 75^3 20.3 / 17.0,
-// 90^3 30.7 / 25.0, 100^3 (354 MB) 43.0 / 45.7).
+// too (two steps per launch, where prefer_pair refuses them by bgk_set_launch;
+// us per step, streaming against plain: FP32 48^3 5.7 / 6.2, 64^3 6.4 / 6.7, 80^3
+// 15.0 / 12.0, 100^3 25.0 / 20.2, 112^3 30.4 / 23.4, 128^3 (411 MB) 36.0 / 37.9; FP64
+// 64^3 (106 MB) 10.7 / 10.8, 75^3 20.3 / 17.0, 90^3 30.7 / 25.0, 100^3 (354 MB) 43.0 /
+// 45.7).
 inline bool keep_in_cache(size_t bytes) { return bytes >= 80000000 && bytes <= size_t(1) << 28; }
 
 // Point mem[0] and mem[1] (the two lattices) into one region of

@@ -16,11 +16,15 @@ void launch_fused(bgk_handle& h, bool pair)
     const FusedArgs<S> p = fused_args<S>(h, h.cur, h.rest);
     if constexpr (kPairs<S>) {
         if (pair) {
-            // the obstacle forms, the longest to compile, always stream
-            if (!OB && keep_in_cache(lattice_bytes(h)))
-                launch_pair<S, BX, BY, BZ, OB, FM, OB>(p, h.pgrid, h.stream);
-            else
-                launch_pair<S, BX, BY, BZ, OB, FM, true>(p, h.pgrid, h.stream);
+            // obstacle forms always stream: they take the longest to compile,
+            // and a plain-store copy of each would double that
+            if constexpr (!OB) {
+                if (keep_in_cache(lattice_bytes(h))) {
+                    launch_pair<S, BX, BY, BZ, OB, FM, false>(p, h.pgrid, h.stream);
+                    return;
+                }
+            }
+            launch_pair<S, BX, BY, BZ, OB, FM, true>(p, h.pgrid, h.stream);
             return;
         }
     }

@@ -52,8 +52,9 @@ __device__ __forceinline__ void block_sum(double (&v)[NV])
 }
 
 // Second pass: one block folds nblk partials (layout [blk][NV]) in order.
-// `out` is host memory the GPU can write (hipHostMalloc): the totals are there
-// when the stream has been waited for, without a copy of their own.
+// `out` is device memory, or host memory that the GPU can write (hipHostMalloc):
+// the totals are then there when the stream has been waited for, without a
+// copy of their own.
 template <int NV>
 __global__ __launch_bounds__(kRedThreads) void fold_partials(const double* __restrict__ part, int nblk,
                                                              double* __restrict__ out)

@@ -379,7 +379,7 @@ void launch_group(bgks_server::Group& g, const SubBatch& sb, int t, int launch, 
 {
     const BatchSlot<S>* d_slots = static_cast<const BatchSlot<S>*>(g.d_slots);
     if (sb.single >= 0) {
-        // the engine's launch for a driven cavity (engine.hip launch_fused)
+        // the engine's launch for a driven cavity (launch.hpp launch_fused)
         const BatchSlot<S>& sl = static_cast<const BatchSlot<S>*>(g.h_slots)[sb.single];
         FusedArgs<S> p = sl.args[launch & 1];
         p.seed = step_seed(sl.cfg_seed, sl.steps0 + t);
