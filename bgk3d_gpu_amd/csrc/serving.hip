@@ -244,6 +244,7 @@ struct bgks_server {
     double* scratch = nullptr;
     double* hscratch = nullptr;
     std::deque<long long> queue;
+    size_t queued = 0, held = 0;  // request_bytes of the queued and of those that hold a lattice, added up
     std::map<long long, std::unique_ptr<Instance>> all;
     long long next_id = 1;
     int policy = BGKS_ALL_ACTIVE;
@@ -455,6 +456,8 @@ int start(bgks_server& s, Instance& in, size_t off)
 {
     in.off = off;
     in.has_mem = true;
+    s.queued -= in.need;
+    s.held += in.need;
     void* region = static_cast<char*>(s.arena_mem) + off;
     place_lattices(in.h, region);
     ENG_HIP(hipMemsetAsync(region, 0, in.len, s.stream));  // rest state: shifted populations are zero
@@ -513,14 +516,7 @@ int find_room(bgks_server& s, Instance& in, size_t& off, bool& found)
     found = true;
     const size_t room = s.arena.size - s.arena.used();
     if (in.roomy && in.roomy <= room) {
-        size_t left = room - in.roomy;
-        bool fits = true;
-        for (long long id : s.queue) {
-            const size_t need = id != in.id ? s.all.at(id)->need : 0;
-            fits = need <= left;
-            if (!fits) break;
-            left -= need;
-        }
+        const bool fits = s.queued - in.need <= room - in.roomy;
         if (fits && s.arena.alloc(in.roomy, off)) {
             if (int rc = handle_setup(in.h, in.h.cfg)) return rc;
             in.len = in.roomy;
@@ -529,10 +525,7 @@ int find_room(bgks_server& s, Instance& in, size_t& off, bool& found)
     }
     in.len = in.need;
     if (s.arena.alloc(in.need, off)) return 0;
-    size_t held = 0;
-    for (auto& kv : s.all)
-        if (kv.second->has_mem) held += kv.second->need;
-    found = s.arena.size - held >= in.need;
+    found = s.arena.size - s.held >= in.need;
     if (found) {
         if (int rc = gather(s)) return rc;
         found = s.arena.alloc(in.need, off);
@@ -591,6 +584,7 @@ void free_lattice(bgks_server& s, Instance& in)
     }
     if (!in.has_mem) return;
     s.arena.release(in.off, in.len);
+    s.held -= in.need;
     in.has_mem = false;
     in.h.mem[0] = in.h.mem[1] = nullptr;
 }
@@ -748,6 +742,7 @@ int bgks_submit(bgks_server* s, const bgks_request* r, long long* id)
     in->t_submit = clock_now();
     *id = in->id;
     s->queue.push_back(in->id);
+    s->queued += in->need;
     s->all[in->id] = std::move(in);
     return 0;
 }
@@ -927,7 +922,10 @@ int bgks_release(bgks_server* s, long long id)
     if (it == s->all.end()) return fail(BGK_EINVAL, "unknown request %lld", id);
     Instance& in = *it->second;
     if (in.state == BGKS_ACTIVE) return fail(BGK_EBUSY, "request %lld is running", id);
-    if (in.state == BGKS_QUEUED) s->queue.erase(std::find(s->queue.begin(), s->queue.end(), id));
+    if (in.state == BGKS_QUEUED) {
+        s->queue.erase(std::find(s->queue.begin(), s->queue.end(), id));
+        s->queued -= in.need;
+    }
     free_lattice(*s, in);
     s->all.erase(it);
     return 0;

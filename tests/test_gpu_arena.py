@@ -100,3 +100,25 @@ def test_one_step_requests_share_launches(gpu):
             srv.submit(r)
         assert len(srv.advance()) == 2
         assert srv.stats()["launches"] == 10
+
+
+def test_a_released_request_claims_nothing(gpu):
+    """The rows of two steps per launch are taken while every queued request
+    fits beside them: one that was released from the queue, or that ended,
+    counts no longer."""
+    r, big = S.Request(87, 200.0, "f32", 6), S.Request(120, 200.0, "f32", 6)
+    need = S.request_bytes(r)
+    with S.Server(need + S.request_bytes(big), 3) as srv:
+        for turn in range(3):
+            a, b = srv.submit(r), srv.submit(big)
+            if turn:
+                srv.release(b)
+            srv.advance()
+            used = srv.stats()["bytes_used"]
+            assert used > need if turn else used == need + S.request_bytes(big), turn
+            finish(srv, a)
+            if not turn:
+                finish(srv, b)
+            assert srv.stats()["bytes_used"] == 0
+            for rid in (a, b)[:1 if turn else 2]:
+                srv.release(rid)

@@ -49,7 +49,7 @@ def test_fields_from_several_threads(gpu):
 
 
 def test_fields_after_a_refused_handle(gpu):
-    """A lattice that cannot be allocated (17 TB) leaves the other handles of
+    """A lattice that cannot be allocated (19 TB) leaves the other handles of
     the thread as they were."""
     with Engine(Case("ldc", 20, 20, 20, svisc=0.05, u0=0.1), "f32") as eng:
         eng.step(2)
